@@ -182,6 +182,25 @@ int khx_patterned_layer_cached(const double* C, const double* IC, int per_item, 
                                int N, int batch, const double* k0d, double* S, double* W, double* V, double* lam,
                                int* info, double* cache, void* ws, void* stream);
 
+/* The S-matrix of the same layer without its modes (the reference always goes
+ * through eig, khepri/alternative.py:158-195): a rational approximant of the
+ * layer cut into 2^doublings slices, then as many star products of a slab with
+ * itself.
+ * khx_layer_scale: est[b] = |k0d sqrt(eigenvalue of P Q)| / 2 of the largest
+ *   eigenvalue, by power iteration (a few per cent; NaN for a non-finite
+ *   input).  The approximant is exact to FP64 rounding while
+ *   est / 2^doublings <= KHX_LAYER_THETA, so
+ *   doublings = max(0, ceil(log2(est / KHX_LAYER_THETA))).
+ * khx_layer_smatrix: S (batch, 2, 2, n, n), one number of doublings for the
+ *   whole batch.  info[b]: 1 a non-finite entry in P Q (numpy's eig raises),
+ *   -1 a solve met an exact zero pivot, else 0.                            */
+#define KHX_LAYER_THETA 2.75
+int khx_layer_scale(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
+                    int batch, const double* k0d, double* est, void* stream);
+size_t khx_layer_smatrix_ws_bytes(int n, int batch, int doublings);
+int khx_layer_smatrix(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
+                      int batch, const double* k0d, int doublings, double* S, int* info, void* ws, void* stream);
+
 /* Uniform layer of permittivity eps (khepri/layer.py:166-168:
  * khepri/alternative.py:130-156 solve_uniform_layer + build_scatmat) and the
  * half spaces (khepri/layer.py:169-178: khepri/alternative.py:32-56

@@ -31,6 +31,9 @@ SIGNATURES = {
     "khx_patterned_layer_ws_bytes": (_sz, [_i, _i]),
     "khx_patterned_layer": (_i, [_dp, _dp, _i, _dp, _dp, _i, _i, _dp, _dp, _dp, _dp, _dp, _ip, _vp, _vp]),
     "khx_patterned_layer_cached": (_i, [_dp, _dp, _i, _dp, _dp, _i, _i, _dp, _dp, _dp, _dp, _dp, _ip, _dp, _vp, _vp]),
+    "khx_layer_scale": (_i, [_dp, _dp, _i, _dp, _dp, _i, _i, _dp, _dp, _vp]),
+    "khx_layer_smatrix_ws_bytes": (_sz, [_i, _i, _i]),
+    "khx_layer_smatrix": (_i, [_dp, _dp, _i, _dp, _dp, _i, _i, _dp, _i, _dp, _ip, _vp, _vp]),
     "khx_uniform_layer": (_i, [_dp, _dp, _i, _i, _dp, _dp, _dp, _dp, _dp, _dp, _vp]),
     "khx_halfspace": (_i, [_i, _dp, _dp, _i, _i, _dp, _dp, _dp, _dp, _dp, _vp]),
     "khx_redheffer_ws_bytes": (_sz, [_i, _i]),

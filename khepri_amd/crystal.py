@@ -20,7 +20,7 @@ from . import chain, ops
 from .device import default_device
 from .expansion import Expansion, compute_kplanar
 from .extension import ExtendedLayer
-from .layer import Layer, stack_layers
+from .layer import Layer, plan_layers, stack_layers
 
 
 def _bytes_per_item(n, unique, length):
@@ -64,6 +64,7 @@ class Crystal:
         self.S, self._RT = None, None
         self.stacking_matrices, self.stacking_reverse_matrices = [], None
         self.stack_positions = []
+        self._plan = {}
 
     @classmethod
     def from_expansion(cls, expansion, **kwargs):
@@ -236,8 +237,10 @@ class Crystal:
             raise ValueError("fields need the full S-matrix chain (rt_only=False)")
         self.S = None
         self._RT = None
+        if not torch.cuda.is_current_stream_capturing():   # a capture replays the plan of the call before it
+            self._plan = plan_layers([self.layers[name] for name in names], kp_all, wl_all)
         if not rt_only and chunk >= B:
-            Layer.solve_batch_many([self.layers[name] for name in names], kp_all, wl_all)
+            Layer.solve_batch_many([self.layers[name] for name in names], kp_all, wl_all, plan=self._plan)
             self._check_layers(names)
             infos = []
             self.stacking_matrices, self.stacking_reverse_matrices, self.Stot = stack_layers(
@@ -272,7 +275,10 @@ class Crystal:
         """Sources sl of the batch: layer solves, chain, R/T into out[...][sl]."""
         kp_all, wl_all, te_all, tm_all = self._sources_dev
         kp, wl = kp_all[sl], wl_all[sl]
-        Layer.solve_batch_many([self.layers[name] for name in names], kp, wl, rt_only=rt_only)
+        # (an extended layer's plan holds several base sources per source)
+        per = {key: len(s) // self.batch for key, s in self._plan.items()}
+        plan = {key: s[sl.start * per[key]:sl.stop * per[key]] for key, s in self._plan.items()}
+        Layer.solve_batch_many([self.layers[name] for name in names], kp, wl, rt_only=rt_only, plan=plan)
         self._check_layers(names)
         if rt_only:
             c = ops.incident(N, kp, wl, te_all[sl], tm_all[sl], self.epsi)

@@ -52,6 +52,11 @@ size_t patterned_layer_ws_bytes(int n, int batch);
 int patterned_layer(hipStream_t s, const cd* C, const cd* IC, long long cstride, const cd* kx, const cd* ky, int N,
                     int batch, const double* k0d, cd* S, cd* Wout, cd* Vout, cd* lamout, int* info, void* ws,
                     cd* cache);
+int layer_scale(hipStream_t s, const cd* C, const cd* IC, long long cstride, const cd* kx, const cd* ky, int N,
+                int batch, const double* k0d, double* est);
+size_t layer_smatrix_ws_bytes(int n, int batch, int doublings);
+int layer_smatrix(hipStream_t s, const cd* C, const cd* IC, long long cstride, const cd* kx, const cd* ky, int N,
+                  int batch, const double* k0d, int doublings, cd* S, int* info, void* ws);
 int analytic_layer(hipStream_t s, int kind, const cd* kx, const cd* ky, int N, int batch, cd eps,
                    const double* k0d, cd* S, cd* W, cd* V, cd* lam);
 size_t star_ws_bytes(int n, int batch);
@@ -236,6 +241,26 @@ int khx_patterned_layer_cached(const double* C, const double* IC, int per_item, 
   return khx::patterned_layer(as_stream(stream), as_cd(C), as_cd(IC), per_item ? (long long)N * N : 0, as_cd(kx),
                               as_cd(ky), N, batch, k0d, as_cd(S), as_cd(W), as_cd(V), as_cd(lam), info, ws,
                               as_cd(cache));
+}
+
+int khx_layer_scale(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
+                    int batch, const double* k0d, double* est, void* stream) {
+  KHX_ENTRY_BEGIN
+  KHX_REQUIRE(N > 0 && batch >= 0 && k0d && est, "khx_layer_scale: bad arguments");
+  return khx::layer_scale(as_stream(stream), as_cd(C), as_cd(IC), per_item ? (long long)N * N : 0, as_cd(kx),
+                          as_cd(ky), N, batch, k0d, est);
+}
+
+size_t khx_layer_smatrix_ws_bytes(int n, int batch, int doublings) {
+  return khx::layer_smatrix_ws_bytes(n, batch, doublings);
+}
+
+int khx_layer_smatrix(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
+                      int batch, const double* k0d, int doublings, double* S, int* info, void* ws, void* stream) {
+  KHX_ENTRY_BEGIN
+  KHX_REQUIRE(N > 0 && batch >= 0 && k0d && S, "khx_layer_smatrix: bad arguments");
+  return khx::layer_smatrix(as_stream(stream), as_cd(C), as_cd(IC), per_item ? (long long)N * N : 0, as_cd(kx),
+                            as_cd(ky), N, batch, k0d, doublings, as_cd(S), info, ws);
 }
 
 int khx_uniform_layer(const double* kx, const double* ky, int N, int batch, const double* eps_host,

@@ -50,7 +50,15 @@ class ExtendedLayer:
     def chain_item(self):
         return ("dense", self.S)
 
-    def solve_batch(self, kp, wl, ws=None, rt_only=False):
+    def plan(self, kp, wl):
+        """Layer.plan of the base at its own sources, (B Nb,) estimates."""
+        if not isinstance(self.base, Layer) or self.fields:
+            return None
+        kpb, wlb, _ = self._base_sources(kp, wl)
+        self.base.fields = self.fields
+        return self.base.plan(kpb, wlb)
+
+    def solve_batch(self, kp, wl, ws=None, rt_only=False, doublings=None):
         if isinstance(self.base, Layer):
             self.base.fields = self.fields
         kpb, wlb, Nb = self._base_sources(kp, wl)
@@ -67,7 +75,7 @@ class ExtendedLayer:
             self.W = self.V = self.L = None
             self.IC = 1.0
             return
-        self.base.solve_batch(kpb, wlb)
+        self.base.solve_batch(kpb, wlb, doublings=doublings)
         self.info = getattr(self.base, "info", None)
         self.S = ops.joint_subspace(self.base.S, Nb, self.mode, 4)
         if self.fields:

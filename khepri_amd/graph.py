@@ -33,6 +33,11 @@ from __future__ import annotations
 import torch
 
 from . import ops
+from .layer import plan_layers
+
+
+def _same_plan(a, b):
+    return a.keys() == b.keys() and all((a[k] == b[k]).all() for k in a)
 
 
 class _Captured:
@@ -48,6 +53,7 @@ class _Captured:
             with ops.deferred_status([]):
                 self._run()
         torch.cuda.current_stream().wait_stream(side)
+        self.plan = dict(self.cl._plan)
         self.graph = torch.cuda.CUDAGraph()
         self.status = []
         with torch.cuda.graph(self.graph):
@@ -56,6 +62,11 @@ class _Captured:
 
     def _run(self):
         raise NotImplementedError
+
+    def _planned(self):
+        cl = self.cl
+        layers = [cl.layers[name] for name in dict.fromkeys(cl.global_stacking)]
+        return plan_layers(layers, *self.sources[:2])
 
     def update_sources(self, wavelength, te=1.0, tm=1.0, theta=0.0, phi=0.0, kp=None):
         """New sources for the next replays (Crystal.set_source's arguments);
@@ -66,6 +77,10 @@ class _Captured:
             raise ValueError(f"the graph was captured for {self.batch} sources, got {cl.batch}")
         for dst, src in zip(self.sources, (cl._kp, cl._wl, cl._te, cl._tm)):
             dst.copy_(torch.as_tensor(src, device=dst.device))
+        # the captured launches are those of the layers' doubling counts, which
+        # the new sources may change: then the sequence is captured again
+        if not _same_plan(self._planned(), self.plan):
+            self._capture()
 
     def _replay(self, check):
         self.graph.replay()

@@ -155,28 +155,32 @@ class Layer:
         return (self.skind, self.X if self.skind == "prop" else self.S)
 
     @staticmethod
-    def solve_batch_many(layers, kp, wl, rt_only=False):
+    def solve_batch_many(layers, kp, wl, rt_only=False, plan=None):
         """solve_batch for several layers of one expansion.  When all their
         eigenproblems fit one round of the eigen-solver (khx_eig_slots), the
         patterned layers are solved together in one fused call so that they
         share the GPU (a single layer's small batch leaves most CUs idle); the
         bound also keeps the fused workspace within one round's worth of
-        items.  Everything else as solve_batch."""
+        items.  plan: {id(layer): doublings per source}, from plan_layers.
+        Everything else as solve_batch."""
+        plan = plan or {}
         pat = [ly for ly in layers if getattr(ly, "patterned", False)]
         B = kp.shape[0]
         fuse = len(pat) >= 2 and B * len(pat) <= ops.eig_slots(2 * pat[0].expansion.N) and \
             all(ly.expansion is pat[0].expansion for ly in pat) and os.environ.get("KHX_FUSE_LAYERS", "1") == "1"
         if not fuse:
             for ly in layers:
-                ly.solve_batch(kp, wl, rt_only=rt_only)
+                ly.solve_batch(kp, wl, rt_only=rt_only, doublings=plan.get(id(ly)))
             return
         dev = kp.device
         kx, ky = ops.kvectors(pat[0].expansion.g_device(dev), kp, wl)
         k0 = 2 * np.pi / wl
         mats = [ly.convolution_matrices(dev) for ly in pat]
         modes = any(bool(ly.fields) for ly in pat)
+        known = [plan.get(id(ly)) for ly in pat]
         res = ops.patterned_layers_fused([m[0] for m in mats], [m[1] for m in mats], kx, ky,
-                                         [(k0 * ly.depth).contiguous() for ly in pat], modes=modes)
+                                         [(k0 * ly.depth).contiguous() for ly in pat], modes=modes,
+                                         doublings=None if any(d is None for d in known) else np.concatenate(known))
         for ly, (C, IC), (S, (W, V, L), info) in zip(pat, mats, res):
             ly.device = dev
             ly.skind, ly.X = "dense", None
@@ -189,11 +193,21 @@ class Layer:
             if not getattr(ly, "patterned", False):
                 ly.solve_batch(kp, wl, rt_only=rt_only)
 
-    def solve_batch(self, kp, wl, ws=None, rt_only=False):
+    def plan(self, kp, wl):
+        """Doublings per source (device estimates, (B,)) of this layer's
+        S-matrix, or None where it has no eigenproblem or keeps its modes."""
+        if not self.patterned or self.fields:
+            return None
+        C, IC = self.convolution_matrices(kp.device)
+        kx, ky = ops.kvectors(self.expansion.g_device(kp.device), kp, wl)
+        return ops.layer_scale(C, IC, kx, ky, (2 * np.pi / wl * self.depth).contiguous())
+
+    def solve_batch(self, kp, wl, ws=None, rt_only=False, doublings=None):
         """S-matrix for a batch.  With rt_only (R/T wanted, no fields), layers of
         the gap medium are kept as their exact structure instead of a dense S:
         a uniform eps = 1 layer as its propagation factors X ("prop"), an
-        eps = 1 half space as the identity S-matrix ("identity")."""
+        eps = 1 half space as the identity S-matrix ("identity").
+        doublings: as ops.patterned_layer takes them."""
         dev = kp.device
         self.device = dev
         kx, ky = ops.kvectors(self.expansion.g_device(dev), kp, wl)
@@ -217,7 +231,8 @@ class Layer:
         if self.patterned:
             C, IC = self.convolution_matrices(dev)
             k0d = (k0 * self.depth).contiguous()
-            self.S, (W, V, L), self.info = ops.patterned_layer(C, IC, kx, ky, k0d, modes=modes, ws=ws)
+            self.S, (W, V, L), self.info = ops.patterned_layer(C, IC, kx, ky, k0d, modes=modes, ws=ws,
+                                                                   doublings=doublings)
             self.C = C
             self.IC = IC if modes else None
         elif self.formulation == Formulation.UNIFORM:
@@ -236,6 +251,31 @@ class Layer:
             raise NotImplementedError(f"formulation {self.formulation}")
         self.W, self.V, self.L = (W, V, L) if modes else (None, None, None)
         self.kx, self.ky = (kx, ky) if modes else (None, None)
+
+
+_PLAN_SOURCES = 16384
+
+
+def plan_layers(layers, kp, wl):
+    """{id(layer): doublings per source} for the layers of a stack whose
+    S-matrices are formed without modes, over all sources of a solve: one
+    estimate launch per layer and slice of sources, one host synchronisation
+    at the end (none between the chunks of the solve)."""
+    if ops.layer_route_is_modal():
+        return {}
+    est = {}
+    for ly in layers:
+        planned = getattr(ly, "plan", None)
+        if planned is not None:
+            parts = [planned(kp[c:c + _PLAN_SOURCES], wl[c:c + _PLAN_SOURCES])
+                     for c in range(0, kp.shape[0], _PLAN_SOURCES)]
+            if parts[0] is not None:
+                est[id(ly)] = torch.cat(parts)
+    if not est:
+        return {}
+    sizes = [len(v) for v in est.values()]
+    counts = ops.doublings_of(torch.cat(list(est.values())))
+    return dict(zip(est, np.split(counts, np.cumsum(sizes)[:-1])))
 
 
 def scattering_identity(B, n, device):

@@ -8,6 +8,8 @@ exceptions the reference's numpy calls raise.
 """
 from __future__ import annotations
 
+import os
+
 import numpy as np
 import torch
 
@@ -310,11 +312,107 @@ def eig(A, overwrite_a=False):
     return lam, W, info
 
 
-def patterned_layer(C, IC, kx, ky, k0d, modes=False, ws=None, cache=None):
+# The slice of a layer may be this thick (|k0 d sqrt(eigenvalue)| / 2): up to
+# here the [13/13] approximant of khx_layer_smatrix is exact to FP64 rounding
+# (khx.h: KHX_LAYER_THETA).
+LAYER_THETA = 2.75
+# Layers that need more doublings go through the eigensolver, whose work does
+# not grow with the depth: each doubling is 37 n^3 operations.
+LAYER_MAX_DOUBLINGS = 12
+# switches that choose something inside the modal route select that route
+_MODAL_KNOBS = ("KHX_EIG_ITMAX", "KHX_LAYER_WINV", "KHX_LAYER_AINV", "KHX_LAYER_VIDENT")
+
+
+def layer_route_is_modal():
+    """True when the environment asks for S-matrices through the eigensolver."""
+    return os.environ.get("KHX_LAYER_MODES", "0") == "1" or any(k in os.environ for k in _MODAL_KNOBS)
+
+
+def layer_scale(C, IC, kx, ky, k0d):
+    """|k0 d sqrt(eigenvalue of P Q)| / 2 of the largest eigenvalue, (B,) on the device."""
+    lib = _lib.load()
+    B, N = kx.shape
+    est = torch.empty(B, dtype=RDT, device=kx.device)
+    C, IC = C.contiguous(), IC.contiguous()
+    check(lib.khx_layer_scale(_p(C), _p(IC), int(C.dim() == 3), _p(kx), _p(ky), N, B, _p(k0d), _p(est), _stream()),
+          "khx_layer_scale")
+    return est
+
+
+def doublings_of(est):
+    """Doublings per item (int array on the host) for layer_scale's estimates;
+    -1 for the items that go through the eigensolver.  A host synchronisation."""
+    with np.errstate(all="ignore"):
+        e = est.cpu().numpy() / LAYER_THETA
+        s = np.where(e > 1.0, np.ceil(np.log2(np.where(e > 1.0, e, 1.0))), 0.0)   # NaN: 0, flagged by the kernel
+    return np.where(s > LAYER_MAX_DOUBLINGS, -1, s).astype(np.int64)
+
+
+def _layer_smatrix(C, IC, kx, ky, k0d, doublings, S, info):
+    lib = _lib.load()
+    B, N = kx.shape
+    ws = _ws(lib.khx_layer_smatrix_ws_bytes(2 * N, B, doublings), kx.device)
+    check(lib.khx_layer_smatrix(_p(C), _p(IC), int(C.dim() == 3), _p(kx), _p(ky), N, B, _p(k0d), doublings, _p(S),
+                                _p(info), _p(ws), _stream()), "khx_layer_smatrix")
+
+
+def layer_smatrix(C, IC, kx, ky, k0d, doublings):
+    """(S (B, 2, 2, n, n), status words) of a patterned layer without its
+    modes; doublings: int array (B,) as doublings_of gives it.  The items of
+    one count are solved together, so an item's result does not depend on the
+    batch it comes in."""
+    B, N = kx.shape
+    n = 2 * N
+    dev = kx.device
+    S = torch.empty((B, 2, 2, n, n), dtype=CDT, device=dev)
+    info = torch.empty(B, dtype=torch.int32, device=dev)
+    counts = np.unique(doublings)
+    for s in counts:
+        if len(counts) == 1:
+            args, Sg, ig = (C, IC, kx, ky, k0d), S, info
+        else:
+            idx = torch.as_tensor(np.nonzero(doublings == s)[0], device=dev)
+            Cg, ICg = (C[idx], IC[idx]) if C.dim() == 3 else (C, IC)
+            args = (Cg, ICg, kx[idx], ky[idx], k0d[idx])
+            Sg = torch.empty((len(idx), 2, 2, n, n), dtype=CDT, device=dev)
+            ig = torch.empty(len(idx), dtype=torch.int32, device=dev)
+        if s < 0:
+            Sm, _, im = _modal_layer(*args)
+            Sg.copy_(Sm)
+            ig.copy_(im)
+        else:
+            _layer_smatrix(*args, int(s), Sg, ig)
+        if len(counts) > 1:
+            S[idx] = Sg
+            info[idx] = ig
+    return S, info
+
+
+def patterned_layer(C, IC, kx, ky, k0d, modes=False, ws=None, cache=None, doublings=None):
     """S (B, 2, 2, n, n) of a patterned layer; (W, V, lam) too when modes.
     C, IC: (N, N) shared by the batch or (B, N, N) one per item.  cache: a
     (B, 9, n, n) complex tensor that receives the solves' results for
-    patterned_layer_bwd (khx_patterned_layer_cached)."""
+    patterned_layer_bwd (khx_patterned_layer_cached).
+
+    Without modes and cache the S-matrix is formed directly
+    (khx_layer_smatrix); doublings: the items' counts if the caller has them
+    (doublings_of(layer_scale(...))), else they are determined here, with a
+    host synchronisation -- which a stream capture does not allow, so a
+    captured call without them goes through the eigensolver."""
+    if not modes and cache is None and not layer_route_is_modal():
+        C, IC = C.contiguous(), IC.contiguous()
+        if C.dim() == 3 and (C.shape[0] != kx.shape[0] or IC.shape[0] != kx.shape[0]):
+            raise ValueError("per-item convolution matrices must match the batch")
+        if doublings is None and not torch.cuda.is_current_stream_capturing():
+            doublings = doublings_of(layer_scale(C, IC, kx, ky, k0d))
+        if doublings is not None:
+            S, info = layer_smatrix(C, IC, kx, ky, k0d, doublings)
+            return S, (None, None, None), info
+    return _modal_layer(C, IC, kx, ky, k0d, modes, ws, cache)
+
+
+def _modal_layer(C, IC, kx, ky, k0d, modes=False, ws=None, cache=None):
+    """patterned_layer through the eigen-decomposition of P Q."""
     lib = _lib.load()
     B, N = kx.shape
     n = 2 * N
@@ -378,10 +476,9 @@ def convmat_islands(islands, eps_host, pw, reciprocal, sigma, device):
     return C
 
 
-def patterned_layers_fused(Cs, ICs, kx, ky, k0ds, modes=False, cache=False):
+def patterned_layers_fused(Cs, ICs, kx, ky, k0ds, modes=False, cache=False, doublings=None):
     """patterned_layer for several layers over the same sources in one call:
-    item l*B + b is layer l at source b, so the eigen-solver and every other
-    stage runs once over L*B items (a small batch of one layer leaves most CUs
+    item l*B + b is layer l at source b, so every stage runs once over L*B items (a small batch of one layer leaves most CUs
     idle).  Returns one (S, (W, V, lam), info) per layer, as views; with
     cache, one (S, (W, V, lam), info, cache) per layer (cache: the
     patterned_layer_bwd intermediates, (B, 9, n, n))."""
@@ -394,7 +491,7 @@ def patterned_layers_fused(Cs, ICs, kx, ky, k0ds, modes=False, cache=False):
     kyl = ky.repeat(L, 1)
     k0dl = torch.cat([k.reshape(B) for k in k0ds])
     cb = torch.empty((L * B, 9, n, n), dtype=CDT, device=kx.device) if cache else None
-    S, (W, V, lam), info = patterned_layer(C, IC, kxl, kyl, k0dl, modes=modes, cache=cb)
+    S, (W, V, lam), info = patterned_layer(C, IC, kxl, kyl, k0dl, modes=modes, cache=cb, doublings=doublings)
     out = []
     for l in range(L):
         sl = slice(l * B, (l + 1) * B)

@@ -1,0 +1,140 @@
+"""Patterned-layer S-matrices formed without modes (khx_layer_smatrix) against
+the oracle's modal S-matrix, over the forms the entry point takes: harmonic
+counts from 1, thin slabs (no doubling) to thick ones (several), lossless,
+lossy and metallic maps, evanescent and complex in-plane wave vectors, shared
+and per-item convolution matrices, batches whose items need different counts.
+
+Tolerance: the oracle's modal formula loses up to cond(W) ~ 1e5 over FP64's
+rounding on these layers, so both sides agree to 1e-10 of the largest entry."""
+import numpy as np
+import pytest
+
+from khepri_amd import workloads as W
+from oracle import rcwa
+
+TOL = 1e-10
+
+
+def oracle_s(eps, pw, lattice, kp, wl, depth):
+    g = rcwa.g_vectors(pw, rcwa.lattice_matrix(lattice))
+    kx, ky, _ = rcwa.k_vectors(g, kp, wl)
+    w, v, lam = rcwa.structured_layer_modes(kx, ky, rcwa.convolution_matrix(eps, pw))
+    w0, v0 = rcwa.free_space_eigenmodes(kx, ky)
+    return rcwa.build_scatmat(w, v, w0, v0, lam, depth, 2 * np.pi / wl)
+
+
+def make_layer(eps, pw, lattice, depth):
+    from khepri_amd import Crystal
+    from khepri_amd.layer import Layer
+    return Layer.pixmap(Crystal(pw, lattice=lattice).expansion, eps, depth)
+
+
+LOSSY = W.disc_pixmap(64, 9.0, 0.3, 2.0) * (1 - 0.02j)
+METAL = W.disc_pixmap(64, 1.0 + 0j, 0.3, -12.0 - 1.0j)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pw,lattice,eps,depth,wl,kp", [
+    ((1, 1), "square", W.disc_pixmap(), 0.4, 1.8, (0.3, 0.1)),
+    ((3, 1), "square", W.disc_pixmap(), 0.01, 1.8, (0.0, 0.0)),
+    ((3, 3), "hexagonal", LOSSY, 0.4, 1.6, (0.5, -0.2)),
+    ((5, 5), "square", W.disc_pixmap(), 0.55, 2.0, (0.9, 0.4)),
+    ((5, 5), "square", METAL, 0.3, 1.8, (0.9, 0.4)),
+    ((5, 7), "square", LOSSY, 6.0, 1.7, (0.2, 0.7)),
+    ((5, 5), "square", W.disc_pixmap(), 0.55, 2.0, (4.0, 1.0)),
+    ((5, 5), "square", LOSSY, 0.55, 2.0, (0.8 + 0.2j, 0.1)),
+    ((9, 9), "square", W.disc_pixmap(), 0.55, 1.9, (0.7, 0.3)),
+])
+def test_matches_modal_oracle(gpu, pw, lattice, eps, depth, wl, kp):
+    ref = oracle_s(eps, pw, lattice, kp, wl, depth)
+    ly = make_layer(eps, pw, lattice, depth)
+    ly.solve(np.array(kp), wl)
+    assert int(ly.info[0]) == 0
+    assert np.abs(ly.S[0].cpu().numpy() - ref).max() <= TOL * np.abs(ref).max()
+
+
+@pytest.mark.gpu
+def test_items_of_different_counts_match_single_solves(gpu):
+    """Per-item convolution matrices and depths from 0.02 to 30: the counts
+    differ inside the batch; each item is what it is on its own, to the last
+    bit where the batch does not change the kernels (3 x 3 harmonics)."""
+    import torch
+    from khepri_amd import ops
+    pw, wl = (3, 3), 1.7
+    depths = np.array([0.02, 30.0, 0.5, 4.0, 0.5])
+    lys = [make_layer(W.disc_pixmap(64, 4.0 + k, 0.3, 1.0), pw, "square", d) for k, d in enumerate(depths)]
+    mats = [ly.convolution_matrices(gpu) for ly in lys]
+    C, IC = (torch.stack([m[q] for m in mats]) for q in (0, 1))
+    kp = torch.as_tensor(np.tile([[0.4 + 0j, 0.2]], (5, 1)), device=gpu)
+    wls = torch.full((5,), wl, dtype=torch.float64, device=gpu)
+    kx, ky = ops.kvectors(lys[0].expansion.g_device(gpu), kp, wls)
+    k0d = 2 * np.pi / wls * torch.as_tensor(depths, device=gpu)
+    counts = ops.doublings_of(ops.layer_scale(C, IC, kx, ky, k0d))
+    assert len(set(counts.tolist())) >= 3
+    S, _, info = ops.patterned_layer(C, IC, kx, ky, k0d)
+    assert (info.cpu().numpy() == 0).all()
+    for k, ly in enumerate(lys):
+        ly.solve(np.array([0.4, 0.2]), wl)
+        assert torch.equal(ly.S[0], S[k])
+        ref = oracle_s(np.asarray(ly.epsilon), pw, "square", (0.4, 0.2), wl, depths[k])
+        assert np.abs(S[k].cpu().numpy() - ref).max() <= TOL * np.abs(ref).max()
+
+
+@pytest.mark.gpu
+def test_depths_beyond_the_doublings_go_through_the_eigensolver(gpu):
+    eps = W.disc_pixmap(64, 4.0, 0.3, 2.0) * (1 - 0.01j)
+    ly = make_layer(eps, (3, 3), "square", 9000.0)
+    ly.solve(np.array([0.3, 0.2]), 1.9)
+    ref = oracle_s(eps, (3, 3), "square", (0.3, 0.2), 1.9, 9000.0)
+    assert np.abs(ly.S[0].cpu().numpy() - ref).max() <= 1e-7 * np.abs(ref).max()   # k0 d = 3e4
+
+
+@pytest.mark.gpu
+def test_non_finite_input_raises_and_rayleigh_order_gives_nan(gpu):
+    """As through the eigensolver: a NaN in k raises LinAlgError; an order
+    whose kz is exactly 0 (wavelength = pitch, normal incidence) gives NaN."""
+    from khepri_amd import ops
+    ly = make_layer(W.disc_pixmap(), (3, 3), "square", 0.5)
+    ly.solve(np.array([np.nan, 0.0]), 1.9)
+    with pytest.raises(np.linalg.LinAlgError):
+        ops.raise_on_info(ly.info, "layer")
+    ly.solve(np.array([0.0, 0.0]), 1.0)
+    assert not np.isfinite(ly.S.cpu().numpy()).any()
+
+
+@pytest.mark.gpu
+def test_graph_recaptures_when_the_counts_change(gpu):
+    """New sources of a captured solve whose layers need another number of
+    doublings: the replay still equals the eager call bit for bit."""
+    from khepri_amd import Crystal
+    from khepri_amd.graph import SolveGraph
+
+    def crystal():
+        cl = Crystal((3, 3))
+        cl.add_layer_pixmap("P", W.disc_pixmap(64, 9.0, 0.3, 1.0), 0.6)
+        cl.set_device(["P"], False)
+        return cl
+    cl = crystal()
+    cl.set_source(np.array([1.9, 2.0]), 1.0, 0.0)
+    g = SolveGraph(cl)
+    before = {k: v.copy() for k, v in g.plan.items()}
+    kp = np.array([[12.0, 9.0], [13.0, 8.0]])      # far evanescent: larger |K|
+    g.update_sources(np.array([1.9, 2.0]), 1.0, 0.0, kp=kp)
+    assert any((before[k] != g.plan[k]).any() for k in before)
+    for _ in range(2):
+        R, T = g.replay()
+        ref = crystal()
+        ref.set_source(np.array([1.9, 2.0]), 1.0, 0.0, kp=kp)
+        ref.solve()
+        Rr, Tr = ref.poynting_flux_end()
+        np.testing.assert_array_equal(R, Rr)
+        np.testing.assert_array_equal(T, Tr)
+
+
+def test_doubling_rule():
+    import torch
+    from khepri_amd import ops
+    t = ops.LAYER_THETA
+    est = torch.tensor([0.0, t, t * 1.001, 2 * t, 2.001 * t, t * 2.0 ** 12, t * 2.0 ** 12 * 1.001, float("nan"),
+                        float("inf")], dtype=torch.float64)
+    assert ops.doublings_of(est).tolist() == [0, 0, 1, 1, 2, 12, -1, 0, -1]
