@@ -122,6 +122,12 @@ int khx_convmat(const double* eps, int is_complex, int nx, int ny, int P, int Q,
  * info[b] = k+1 when the k-th pivot is exactly zero (numpy: LinAlgError). */
 int khx_zgesv(int n, int nrhs, double* A, double* B, int batch, int* info, void* stream);
 
+/* The same with scratch (khx_zgesv_ws_bytes): blocked Gauss-Jordan on the
+ * matrix cores in two launches for n <= 512, where A holds no LU factors
+ * afterwards; khx_zgesv beyond.                                            */
+size_t khx_zgesv_ws_bytes(int n, int batch);
+int khx_zgesv_ws(int n, int nrhs, double* A, double* B, int batch, int* info, void* ws, void* stream);
+
 /* Strided-batched complex GEMM C = alpha A B + beta C (numpy matmul as used
  * throughout khepri/alternative.py).  Item b of A is the M x K row-major
  * matrix at A + b*strideA with row stride lda (complex elements); a batch
@@ -219,6 +225,10 @@ int khx_halfspace(int side, const double* kx, const double* ky, int N, int batch
 size_t khx_redheffer_ws_bytes(int n, int batch);
 int khx_redheffer(const double* SA, int a_bcast, const double* SB, int b_bcast, int n, int batch, double* S,
                   int* info, void* ws, void* stream);
+/* The same with both solves in one batch of khx_zgesv_ws's kind (two launches,
+ * Gauss-Jordan); where fields are read from the chain use khx_redheffer.   */
+int khx_redheffer_gj(const double* SA, int a_bcast, const double* SB, int b_bcast, int n, int batch, double* S,
+                     int* info, void* ws, void* stream);
 
 /* Reflected and transmitted power (khepri/crystal.py:363-396
  * poynting_flux_end, with khepri/alternative.py:101-128 incident and

@@ -21,6 +21,8 @@ SIGNATURES = {
     "khx_convmat_ws_bytes": (_sz, [_i, _i, _i]),
     "khx_convmat": (_i, [_dp, _i, _i, _i, _i, _i, _i, _dp, _vp, _vp]),
     "khx_zgesv": (_i, [_i, _i, _dp, _dp, _i, _ip, _vp]),
+    "khx_zgesv_ws_bytes": (_sz, [_i, _i]),
+    "khx_zgesv_ws": (_i, [_i, _i, _dp, _dp, _i, _ip, _vp, _vp]),
     "khx_zgemm": (_i, [_i, _i, _i, _dp, _dp, _i, C.c_longlong, _dp, _i, C.c_longlong, _dp, _dp, _i, C.c_longlong,
                        _i, _vp]),
     "khx_eig_ws_bytes": (_sz, [_i, _i]),
@@ -38,6 +40,7 @@ SIGNATURES = {
     "khx_halfspace": (_i, [_i, _dp, _dp, _i, _i, _dp, _dp, _dp, _dp, _dp, _vp]),
     "khx_redheffer_ws_bytes": (_sz, [_i, _i]),
     "khx_redheffer": (_i, [_dp, _i, _dp, _i, _i, _i, _dp, _ip, _vp, _vp]),
+    "khx_redheffer_gj": (_i, [_dp, _i, _dp, _i, _i, _i, _dp, _ip, _vp, _vp]),
     "khx_poynting_ws_bytes": (_sz, [_i, _i]),
     "khx_poynting": (_i, [_dp, _i, _dp, _dp, _dp, _dp, _dp, _dp, _dp, _i, _dp, _dp, _dp, _dp, _vp, _vp]),
     "khx_incident": (_i, [_i, _dp, _dp, _dp, _dp, _dp, _i, _dp, _vp]),

@@ -9,9 +9,10 @@ Stot = S_1 * R_2, R_j = S_j * R_{j+1} (Redheffer products, khepri/alternative.py
     Stot11 c = S11_1 c + S12_1 D_1^-1 R11_2 S21_1 c
     Stot21 c = R21_2 F_1^-1 S21_1 c,  F^-1 y = y + S22 D^-1 R11 y   (push-through)
 
-so each junction costs one GEMM and one LU (plus one solve and two GEMMs to
-build R11_j when more junctions follow) and the rest is matrix-vector work --
-the same R and T as the full chain, without forming the other three blocks.
+so each junction costs one GEMM and one solve -- with a single right-hand side
+at the first junction, with Z_j = D_j^-1 R11_{j+1} and two more GEMMs for R11_j
+where more junctions follow -- and the rest is matrix-vector work: the same R
+and T as the full chain, without forming the other three blocks.
 
 Layers whose medium is the gap medium (uniform eps = 1: S = [[0, X], [X, 0]])
 fold into a neighbour as diagonal scalings, and eps = 1 half spaces are the
@@ -80,33 +81,30 @@ def rt_amplitudes(items, c):
     if m == 1:
         S = seq[0]
         return _mv(S[:, 0, 0], c), _mv(S[:, 1, 0], c), []
-    # right-to-left: R11 of every right sub-stack and the LU of each junction
-    R11 = [None] * m
-    LU = [None] * m
-    R11[m - 1] = seq[m - 1][:, 0, 0]
+    # right-to-left: R11 of every right sub-stack and Z_j = D_j^-1 R11_{j+1}
+    R11 = seq[m - 1][:, 0, 0]
+    Z = [None] * m
     infos = []
-    for j in range(m - 2, -1, -1):
+    for j in range(m - 2, 0, -1):
         Sj = seq[j]
-        P = ops.matmul(R11[j + 1], Sj[:, 1, 1])
-        D = ops.identity_minus(P, out=P)            # temporaries: factored in place
-        if j >= 1:  # factor D_j and solve for R11_{j+1} S21_j in the same pass
-            lu, piv, info, Y = ops.lu_factor_solve(D, ops.matmul(R11[j + 1], Sj[:, 1, 0]),
-                                                   overwrite_a=True, overwrite_b=True)
-            R11[j] = ops.matmul(Sj[:, 0, 1], Y, beta=1.0, C=Sj[:, 0, 0].clone())
-        else:
-            lu, piv, info = ops.lu_factor(D, overwrite_a=True)
+        P = ops.matmul(R11, Sj[:, 1, 1])
+        Z[j], info = ops.solve_conditioned(ops.identity_minus(P, out=P), R11, overwrite_a=True)
         infos.append(info)
-        LU[j] = (lu, piv)
+        R11 = ops.matmul(Sj[:, 0, 1], ops.matmul(Z[j], Sj[:, 1, 0]), beta=1.0, C=Sj[:, 0, 0].clone())
     # left-to-right vector pass
     S1 = seq[0]
     v = _mv(S1[:, 1, 0], c)
-    u = ops.lu_solve(LU[0][0], LU[0][1], _mv(R11[1], v), overwrite_b=True)[..., 0]
+    P = ops.matmul(R11, S1[:, 1, 1])
+    u, info = ops.solve_conditioned(ops.identity_minus(P, out=P), _mv(R11, v).unsqueeze(-1), overwrite_a=True,
+                                    overwrite_b=True)
+    infos.append(info)
+    u = u[..., 0]
     sR = _mv(S1[:, 0, 1], u, add=_mv(S1[:, 0, 0], c))
     y = _mv(S1[:, 1, 1], u, add=v)
     for j in range(1, m - 1):
         Sj = seq[j]
         v = _mv(Sj[:, 1, 0], y)
-        u = ops.lu_solve(LU[j][0], LU[j][1], _mv(R11[j + 1], v), overwrite_b=True)[..., 0]
+        u = _mv(Z[j], v)
         y = _mv(Sj[:, 1, 1], u, add=v)
     sT = _mv(seq[m - 1][:, 1, 0], y)
     return sR, sT, infos

@@ -665,6 +665,29 @@ int zgesv(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* info) {
   return 0;
 }
 
+// KHX_LU_* switches choose something inside the LU paths, so they select those
+static bool lu_switched() {
+  for (const char* k : {"KHX_LU_PATH", "KHX_LU_UNBLOCKED", "KHX_LU_NB", "KHX_LU_RECSOLVE", "KHX_LU_RECFACTOR",
+                        "KHX_LU_PANEL_REG", "KHX_LU_PANEL_TH"})
+    if (getenv(k)) return true;
+  const char* mixed = getenv("KHX_LU_MIXED");
+  return mixed && atoi(mixed) != 0;
+}
+
+int zgesv_ws(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* perm, int* info) {
+  if (batch <= 0 || n <= 0) return 0;
+  if (perm && zgj_fits(n, m) && !lu_switched()) return zgj_solve(s, n, m, A, B, batch, perm, info);
+  if (lu_path(n) == 2 && batch > 65535) {  // the multi-launch LU takes at most 65535 systems per call
+    for (int b0 = 0; b0 < batch; b0 += 65535) {
+      const int nb = batch - b0 < 65535 ? batch - b0 : 65535;
+      KHX_TRY(zgesv(s, n, m, Mat{A.p + b0 * A.stride, A.ld, A.stride}, Mat{B.p + b0 * B.stride, B.ld, B.stride}, nb,
+                    info ? info + b0 : nullptr));
+    }
+    return 0;
+  }
+  return zgesv(s, n, m, A, B, batch, info);
+}
+
 // ======================================================================== elementwise
 // Grid: x over (rows*cols) chunks, y over batch chunks.
 __global__ void zset_identity_kernel(cd* A, int ld, long long sA, int rows, int cols, cd diag,

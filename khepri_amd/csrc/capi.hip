@@ -61,7 +61,7 @@ int analytic_layer(hipStream_t s, int kind, const cd* kx, const cd* ky, int N, i
                    const double* k0d, cd* S, cd* W, cd* V, cd* lam);
 size_t star_ws_bytes(int n, int batch);
 int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, int n, int batch, cd* S,
-         int* info, void* ws);
+         int* info, void* ws, bool gj);
 int poynting(hipStream_t s, const cd* S, long long sS, int N, const double* g, const cd* kp, const double* wl,
              const cd* te, const cd* tm, cd epsi, cd epse, int batch, double* R, double* T, double* Rord,
              double* Tord, cd* ws);
@@ -243,6 +243,15 @@ int khx_patterned_layer_cached(const double* C, const double* IC, int per_item, 
                               as_cd(cache));
 }
 
+size_t khx_zgesv_ws_bytes(int n, int batch) { return (size_t)n * batch * sizeof(int) + 256; }
+
+int khx_zgesv_ws(int n, int nrhs, double* A, double* B, int batch, int* info, void* ws, void* stream) {
+  KHX_ENTRY_BEGIN
+  KHX_REQUIRE(n > 0 && nrhs > 0 && batch >= 0 && ws, "khx_zgesv_ws: bad arguments");
+  return khx::zgesv_ws(as_stream(stream), n, nrhs, khx::Mat{as_cd(A), n, (long long)n * n},
+                       khx::Mat{as_cd(B), nrhs, (long long)n * nrhs}, batch, static_cast<int*>(ws), info);
+}
+
 int khx_layer_scale(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
                     int batch, const double* k0d, double* est, void* stream) {
   KHX_ENTRY_BEGIN
@@ -289,7 +298,17 @@ int khx_redheffer(const double* SA, int a_bcast, const double* SB, int b_bcast, 
   KHX_REQUIRE(S != SA && S != SB, "khx_redheffer: S must not alias an operand");
   const long long s4 = 4ll * n * n;
   return khx::star(as_stream(stream), as_cd(SA), a_bcast ? 0 : s4, as_cd(SB), b_bcast ? 0 : s4, n, batch, as_cd(S),
-                   info, ws);
+                   info, ws, false);
+}
+
+int khx_redheffer_gj(const double* SA, int a_bcast, const double* SB, int b_bcast, int n, int batch, double* S,
+                  int* info, void* ws, void* stream) {
+  KHX_ENTRY_BEGIN
+  KHX_REQUIRE(n > 0 && batch >= 0, "khx_redheffer_gj: bad sizes");
+  KHX_REQUIRE(S != SA && S != SB, "khx_redheffer_gj: S must not alias an operand");
+  const long long s4 = 4ll * n * n;
+  return khx::star(as_stream(stream), as_cd(SA), a_bcast ? 0 : s4, as_cd(SB), b_bcast ? 0 : s4, n, batch, as_cd(S),
+                   info, ws, true);
 }
 
 size_t khx_poynting_ws_bytes(int N, int batch) { return (size_t)3 * 2 * N * sizeof(cd) * batch + 256; }

@@ -30,6 +30,12 @@ int gemm_record(int on, int* shapes, int max_shapes);
 // Solve A X = B (A n x n destroyed, B n x m overwritten); info[b] = first zero pivot (1-based) or 0
 int zgesv(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* info);
 
+// the same with n ints of scratch per item in `perm`: Gauss-Jordan on the matrix
+// cores for orders up to 512 (lu_gj.hip), else zgesv
+int zgesv_ws(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* perm, int* info);
+bool zgj_fits(int n, int m);
+int zgj_solve(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* perm, int* info);
+
 // LU factors with pivots (zgetrf layout) and the solve of their system
 int zgetrf(hipStream_t s, int n, Mat A, int batch, int* ipiv, int* info);
 int zgetrs(hipStream_t s, int n, int m, Mat A, const int* ipiv, Mat B, int batch);

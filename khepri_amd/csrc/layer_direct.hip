@@ -474,7 +474,7 @@ constexpr int DIRECT_ITEMS = 13;
 
 size_t layer_smatrix_ws_bytes(int n, int batch, int doublings) {
   return (size_t)DIRECT_ITEMS * n * n * sizeof(cd) * batch + (size_t)2 * n * sizeof(cd) * batch +
-         (size_t)batch * sizeof(int) * (1 + 2 * (doublings + 2)) + 256;
+         (size_t)batch * sizeof(int) * (1 + 2 * (doublings + 2) + 2 * n) + 256;
 }
 
 int layer_smatrix(hipStream_t s, const cd* C, const cd* IC, long long cstride, const cd* kx, const cd* ky, int N,
@@ -505,10 +505,10 @@ int layer_smatrix(hipStream_t s, const cd* C, const cd* IC, long long cstride, c
   int* bad = reinterpret_cast<int*>(w);
   int* words = bad + batch;
   const int nwords = 2 * (doublings + 2);
-  const cd one = mkc(1.0, 0.0), mone = mkc(-1.0, 0.0), zero = mkc(0.0, 0.0);
+  int* perm = words + (long long)nwords * batch;
+  const cd one = mkc(1.0, 0.0), zero = mkc(0.0, 0.0);
   const Mat mC{const_cast<cd*>(C), N, cstride}, mIC{const_cast<cd*>(IC), N, cstride};
   const double scale = ldexp(1.0, -doublings);
-  (void)mone;
 
   zero_words_kernel<<<dim3((batch + 255) / 256), 256, 0, s>>>(bad, batch);
   KHX_LAUNCH_CHECK();
@@ -536,7 +536,7 @@ int layer_smatrix(hipStream_t s, const cd* C, const cd* IC, long long cstride, c
   slice_systems_kernel<<<tg, 256, 0, s>>>(CS, Cs, G, kx, ky, k0d, scale, N, batch, tiles, A, B);
   KHX_LAUNCH_CHECK();
   const Mat mA{A, n, nn};
-  KHX_TRY(zgesv(s, n, n, mA, Mat{B, n, nn}, 2 * batch, words));
+  KHX_TRY(zgesv_ws(s, n, n, mA, Mat{B, n, nn}, 2 * batch, perm, words));
   cd* B2 = U;
   slice_s_kernel<<<tg, 256, 0, s>>>(B, n, batch, tiles, S, A, B2, doublings > 0);
   KHX_LAUNCH_CHECK();
@@ -546,7 +546,7 @@ int layer_smatrix(hipStream_t s, const cd* C, const cd* IC, long long cstride, c
       doubling_kernel<<<grid_ew(nn * batch), 256, 0, s>>>(S, n, batch, A, B2);
       KHX_LAUNCH_CHECK();
     }
-    KHX_TRY(zgesv(s, n, n, mA, Mat{B2, n, nn}, 2 * batch, words + 2ll * (k + 1) * batch));
+    KHX_TRY(zgesv_ws(s, n, n, mA, Mat{B2, n, nn}, 2 * batch, perm, words + 2ll * (k + 1) * batch));
     KHX_TRY(zgemm(s, n, n, n, one, s12, Mat{B2, n, nn}, zero, Mat{S + 2 * nn, n, 4 * nn}, batch));
     KHX_TRY(zgemm(s, n, n, n, one, s12, Mat{B2 + nn * batch, n, nn}, zero, Mat{S + 3 * nn, n, 4 * nn}, batch));
   }
@@ -555,7 +555,7 @@ int layer_smatrix(hipStream_t s, const cd* C, const cd* IC, long long cstride, c
   KHX_LAUNCH_CHECK();
   gap_systems_kernel<<<grid_ew((long long)n * N * batch), 256, 0, s>>>(S, r1, N, batch, doublings > 0, A, B);
   KHX_LAUNCH_CHECK();
-  KHX_TRY(zgesv(s, n, n, mA, Mat{B, n, nn}, 2 * batch, words + 2ll * (doublings + 1) * batch));
+  KHX_TRY(zgesv_ws(s, n, n, mA, Mat{B, n, nn}, 2 * batch, perm, words + 2ll * (doublings + 1) * batch));
   gap_s_kernel<<<grid_ew(NN * batch), 256, 0, s>>>(B, r1, N, batch, S);
   KHX_LAUNCH_CHECK();
   if (info) {

@@ -2,7 +2,7 @@
 //   D = I - SB11 SA22,  F = I - SA22 SB11
 //   S11 = SA11 + SA12 D^-1 SB11 SA21     S12 = SA12 D^-1 SB12
 //   S21 = SB21 F^-1 SA21                 S22 = SB22 + SB21 F^-1 SA22 SB12
-// Two LU solves with 2n right-hand sides ([SB11 | SB12] and [SA21 | SA22])
+// Two solves with 2n right-hand sides ([SB11 | SB12] and [SA21 | SA22])
 // and eight GEMMs per product, all batched.  S must not alias SA or SB.
 #include "khx_internal.h"
 
@@ -14,11 +14,16 @@ __global__ void star_info_kernel(const int* __restrict__ infos, int batch, int* 
 }
 
 size_t star_ws_bytes(int n, int batch) {
-  return (size_t)8 * n * n * sizeof(cd) * batch + (size_t)2 * batch * sizeof(int) + 256;
+  return (size_t)8 * n * n * sizeof(cd) * batch + (size_t)2 * (n + 1) * batch * sizeof(int) + 256;
 }
 
+// gj: both systems in one batch through the two-launch Gauss-Jordan
+// (zgesv_ws; D and F are well conditioned for passive layers).  The chains that
+// fields are read from keep the LU: the mode amplitudes inside a layer are
+// differences of terms as large as e^{lambda d}, and carry every rounding of the
+// chain magnified as much.
 int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, int n, int batch, cd* S,
-         int* info, void* wsv) {
+         int* info, void* wsv, bool gj) {
   if (batch <= 0) return 0;
   const long long nn = (long long)n * n;
   const cd one = mkc(1.0, 0.0), mone = mkc(-1.0, 0.0), zero = mkc(0.0, 0.0);
@@ -29,6 +34,7 @@ int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, 
   cd* RF = RD + 2 * nn * batch;   // n x 2n
   cd* tmp = RF + 2 * nn * batch;  // n x n
   int* infos = reinterpret_cast<int*>(tmp + nn * batch);
+  int* perm = infos + 2 * (long long)batch;
   auto blk = [&](const cd* base, long long str, int q) { return Mat{const_cast<cd*>(base) + q * nn, n, str}; };
   const Mat A11 = blk(SA, sA, 0), A12 = blk(SA, sA, 1), A21 = blk(SA, sA, 2), A22 = blk(SA, sA, 3);
   const Mat B11 = blk(SB, sB, 0), B12 = blk(SB, sB, 1), B21 = blk(SB, sB, 2), B22 = blk(SB, sB, 3);
@@ -48,8 +54,12 @@ int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, 
   KHX_TRY(zcopy(s, mRD2, B12, n, n, batch));
   KHX_TRY(zcopy(s, mRF, A21, n, n, batch));
   KHX_TRY(zcopy(s, mRF2, A22, n, n, batch));
-  KHX_TRY(zgesv(s, n, 2 * n, mD, mRD, batch, infos));
-  KHX_TRY(zgesv(s, n, 2 * n, mF, mRF, batch, infos + batch));
+  if (gj) {  // (D, F and the right-hand sides follow each other)
+    KHX_TRY(zgesv_ws(s, n, 2 * n, mD, mRD, 2 * batch, perm, infos));
+  } else {
+    KHX_TRY(zgesv(s, n, 2 * n, mD, mRD, batch, infos));
+    KHX_TRY(zgesv(s, n, 2 * n, mF, mRF, batch, infos + batch));
+  }
   // S11 = SA11 + (SA12 X1) SA21
   KHX_TRY(zgemm(s, n, n, n, one, A12, mRD, zero, mT, batch));
   KHX_TRY(zcopy(s, S11, A11, n, n, batch));
@@ -78,7 +88,7 @@ int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, 
 //   [B11bar | B12bar] += D^-H [X1bar | X2bar], Dbar = -D^-H [X1bar | X2bar] [X1 | X2]^H,
 //   and D = I - B11 A22, F = I - A22 B11 pass Dbar, Fbar on to B11 and A22.
 size_t star_bwd_ws_bytes(int n, int batch) {
-  return (size_t)16 * n * n * sizeof(cd) * batch + (size_t)4 * batch * sizeof(int) + 256;
+  return (size_t)16 * n * n * sizeof(cd) * batch + (size_t)(4 + 2 * n) * batch * sizeof(int) + 256;
 }
 
 int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, int n, int batch, const cd* Sbar,
@@ -105,6 +115,7 @@ int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long 
   cd* T1 = take(1);
   cd* T2 = take(1);
   int* infos = reinterpret_cast<int*>(w);
+  int* perm = infos + 4 * (long long)batch;
   auto blk = [&](const cd* base, long long str, int q) { return Mat{const_cast<cd*>(base) + q * nn, n, str}; };
   const Mat A11 = blk(SA, sA, 0), A12 = blk(SA, sA, 1), A21 = blk(SA, sA, 2), A22 = blk(SA, sA, 3);
   const Mat B11 = blk(SB, sB, 0), B12 = blk(SB, sB, 1), B21 = blk(SB, sB, 2), B22 = blk(SB, sB, 3);
@@ -128,8 +139,7 @@ int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long 
   KHX_TRY(zcopy(s, mX2, B12, n, n, batch));
   KHX_TRY(zcopy(s, mRF, A21, n, n, batch));
   KHX_TRY(zcopy(s, mY2, A22, n, n, batch));
-  KHX_TRY(zgesv(s, n, 2 * n, mD, mRD, batch, infos));
-  KHX_TRY(zgesv(s, n, 2 * n, mF, mRF, batch, infos + batch));
+  KHX_TRY(zgesv_ws(s, n, 2 * n, mD, mRD, 2 * batch, perm, infos));
 
   // S11 = A11 + A12 X1 A21, S12 = A12 X2
   KHX_TRY(zcopy(s, a11, G11, n, n, batch));
@@ -152,12 +162,12 @@ int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long 
   KHX_TRY(zgemm(s, n, n, n, one, B21, mY2, zero, mT1, batch));
   KHX_TRY(zgemm_op(s, 2, 0, n, n, n, one, mT1, G22, zero, b12, batch));
   // [X1 | X2] = D^-1 [B11 | B12]
-  KHX_TRY(zgesv(s, n, 2 * n, mDH, mZX, batch, infos + 2 * batch));
+  KHX_TRY(zgesv_ws(s, n, 2 * n, mDH, mZX, batch, perm, infos + 2 * batch));
   KHX_TRY(zcopy(s, b11, mZX, n, n, batch));
   KHX_TRY(zaxpby(s, b12, one, b12, one, mZX2, n, n, batch));
   KHX_TRY(zgemm_op(s, 0, 2, n, n, 2 * n, mone, mZX, mRD, zero, mDb, batch));
   // [Y1 | Y2] = F^-1 [A21 | A22]
-  KHX_TRY(zgesv(s, n, 2 * n, mFH, mZY, batch, infos + 3 * batch));
+  KHX_TRY(zgesv_ws(s, n, 2 * n, mFH, mZY, batch, perm, infos + 3 * batch));
   KHX_TRY(zaxpby(s, a21, one, a21, one, mZY, n, n, batch));
   KHX_TRY(zcopy(s, a22, mZY2, n, n, batch));
   KHX_TRY(zgemm_op(s, 0, 2, n, n, 2 * n, mone, mZY, mRF, zero, mFb, batch));

@@ -300,7 +300,7 @@ def stack_layers(pw, layers, mask, reverse=True, ws=None, infos=None):
     Stot = layers[0].S
     Sls = [Stot if mask[0] else None]
     for keep, layer in zip(mask[1:], layers[1:]):
-        Stot, info = ops.redheffer(Stot, layer.S, ws=ws)
+        Stot, info = ops.redheffer(Stot, layer.S, ws=ws, gj=not reverse)
         if infos is not None:
             infos.append(info)
         Sls.append(Stot if keep else None)

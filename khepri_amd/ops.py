@@ -152,6 +152,20 @@ def solve(A, B, overwrite_a=False, overwrite_b=False):
     return X, info
 
 
+def solve_conditioned(A, B, overwrite_a=False, overwrite_b=False):
+    """solve for well-conditioned systems (khx_zgesv_ws: two launches, Gauss-
+    Jordan): the forward error is that of an LU, the residual of an
+    ill-conditioned system may be larger."""
+    lib = _lib.load()
+    Af = _owned(A, overwrite_a)
+    X = _owned(B, overwrite_b)
+    b, n, m = X.shape
+    info = torch.empty(b, dtype=torch.int32, device=A.device)
+    ws = _ws(lib.khx_zgesv_ws_bytes(n, b), A.device)
+    check(lib.khx_zgesv_ws(n, m, _p(Af), _p(X), b, _p(info), _p(ws), _stream()), "khx_zgesv_ws")
+    return X, info
+
+
 def inverse(A):
     b, n, _ = A.shape
     I = torch.eye(n, dtype=CDT, device=A.device).expand(b, n, n).contiguous()
@@ -523,7 +537,10 @@ def analytic_layer(kind, kx, ky, eps, k0d=None, modes=False):
     return S, (W, V, lam)
 
 
-def redheffer(SA, SB, out=None, ws=None):
+def redheffer(SA, SB, out=None, ws=None, gj=False):
+    """SA * SB, with its status words; gj: the two solves through
+    khx_zgesv_ws's Gauss-Jordan in one batch -- for chains that only R, T or S
+    are read from (a chain that fields are read from keeps the LU)."""
     lib = _lib.load()
     ab = SA.dim() == 4
     bb = SB.dim() == 4
@@ -536,8 +553,8 @@ def redheffer(SA, SB, out=None, ws=None):
     if ws is None or ws.numel() < need:
         ws = _ws(need, dev)
     SA, SB = SA.contiguous(), SB.contiguous()   # kept alive until the launch is enqueued
-    check(lib.khx_redheffer(_p(SA), int(ab), _p(SB), int(bb), n, B, _p(S), _p(info),
-                            _p(ws), _stream()), "khx_redheffer")
+    fn = lib.khx_redheffer_gj if gj else lib.khx_redheffer
+    check(fn(_p(SA), int(ab), _p(SB), int(bb), n, B, _p(S), _p(info), _p(ws), _stream()), "khx_redheffer")
     return S, info
 
 

@@ -1,0 +1,68 @@
+"""Two-launch Gauss-Jordan solve (khx_zgesv_ws, lu_gj.hip) against numpy, at the
+orders where its tiling changes: one panel and less (1, 15, 16, 17), the edges of
+the wavefront tilings (64/65, 128/129, 192/193, 256/257, 384/385, 512) and
+beyond them (the LU path), right-hand sides around the 16- and 32-column strips,
+batches below and above the strip rule.
+
+Tolerance: forward error <= 1e-16 * n * cond(A) * 64 (growth of partial
+pivoting on random matrices stays far below 64)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _solve(A, B, gpu):
+    import torch
+    from khepri_amd import ops
+    X, info = ops.solve_conditioned(torch.as_tensor(A, device=gpu), torch.as_tensor(B, device=gpu))
+    return X.cpu().numpy(), info.cpu().numpy()
+
+
+@pytest.mark.parametrize("n,m,batch", [
+    (1, 1, 3), (2, 5, 1), (15, 16, 2), (16, 17, 2), (17, 1, 2), (31, 33, 3), (50, 50, 70), (64, 31, 2), (65, 64, 2),
+    (98, 97, 130), (128, 16, 2), (129, 40, 2), (162, 162, 3), (162, 162, 90), (192, 15, 2), (193, 33, 2),
+    (256, 20, 2), (257, 50, 2), (338, 100, 2), (384, 32, 1), (385, 17, 1), (512, 48, 1), (513, 70, 1)])
+def test_orders_and_strips(gpu, n, m, batch):
+    rng = np.random.default_rng(n * 1000 + m)
+    A = rng.normal(size=(batch, n, n)) + 1j * rng.normal(size=(batch, n, n))
+    B = rng.normal(size=(batch, n, m)) + 1j * rng.normal(size=(batch, n, m))
+    X, info = _solve(A, B, gpu)
+    assert (info == 0).all()
+    for b in {0, batch // 2, batch - 1}:
+        ref = np.linalg.solve(A[b], B[b])
+        err = np.linalg.norm(X[b] - ref) / np.linalg.norm(ref)
+        assert err <= 64e-16 * n * np.linalg.cond(A[b]), (b, err)
+
+
+@pytest.mark.parametrize("n", [18, 50, 130])
+def test_pivots_far_from_the_diagonal(gpu, n):
+    """A reversed diagonal with small noise: every pivot row lies in another
+    wavefront's rows than its column; scales from 1e-200 to 1e200."""
+    rng = np.random.default_rng(n)
+    A = (rng.normal(size=(4, n, n)) + 1j * rng.normal(size=(4, n, n))) * 1e-3
+    A[:, np.arange(n), n - 1 - np.arange(n)] += 2.0 + 1.0j
+    scale = np.array([1.0, 1e-200, 1e200, 1e-30])[:, None, None]
+    B = rng.normal(size=(4, n, 7)) + 1j * rng.normal(size=(4, n, 7))
+    X, info = _solve(A * scale, B, gpu)
+    assert (info == 0).all()
+    for b in range(4):
+        ref = np.linalg.solve(A[b], B[b])
+        assert np.abs(X[b] * scale[b] - ref).max() <= 64e-16 * n * np.linalg.cond(A[b]) * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("n", [3, 50, 162])
+def test_singular_and_nan_items(gpu, n):
+    """An exactly singular item is reported with its first zero pivot and leaves
+    the others alone; a NaN item gives NaN."""
+    rng = np.random.default_rng(3)
+    A = rng.normal(size=(4, n, n)) + 1j * rng.normal(size=(4, n, n))
+    B = rng.normal(size=(4, n, 4)) + 0j
+    A[1, :, n - 1] = 0.0
+    A[2, n // 2, 0] = np.nan
+    X, info = _solve(A, B, gpu)
+    assert info[0] == 0 and info[3] == 0 and info[1] == n
+    assert np.isnan(X[2]).all() and not np.isfinite(X[1]).any()
+    for b in (0, 3):
+        ref = np.linalg.solve(A[b], B[b])
+        assert np.linalg.norm(X[b] - ref) <= 64e-16 * n * np.linalg.cond(A[b]) * np.linalg.norm(ref)
