@@ -13,6 +13,32 @@ __global__ void star_info_kernel(const int* __restrict__ infos, int batch, int* 
   if (b < batch) out[b] = infos[b] ? infos[b] : infos[batch + b];
 }
 
+// What the star product's GEMMs and solves start from, in one pass: D = F = I,
+// RD = [SB11 | SB12], RF = [SA21 | SA22], S11 = SA11, S22 = SB22.  (Eight small
+// launches otherwise, a third of a small batch's star product.)
+__global__ void star_prep_kernel(const cd* __restrict__ SA, long long sA, const cd* __restrict__ SB, long long sB,
+                                 int n, int batch, cd* __restrict__ D, cd* __restrict__ F, cd* __restrict__ RD,
+                                 cd* __restrict__ RF, cd* __restrict__ S) {
+  const long long nn = (long long)n * n, total = nn * batch;
+  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
+       e += (long long)gridDim.x * blockDim.x) {
+    const long long b = e / nn, o = e % nn;
+    const int r = (int)(o / n), c = (int)(o % n);
+    const cd* a = SA + b * sA + o;
+    const cd* bb = SB + b * sB + o;
+    const cd d = mkc(r == c ? 1.0 : 0.0, 0.0);
+    D[e] = d;
+    F[e] = d;
+    const long long q = b * 2 * nn + (long long)r * 2 * n + c;
+    RD[q] = bb[0];
+    RD[q + n] = bb[nn];
+    RF[q] = a[2 * nn];
+    RF[q + n] = a[3 * nn];
+    S[b * 4 * nn + o] = a[0];
+    S[b * 4 * nn + 3 * nn + o] = bb[3 * nn];
+  }
+}
+
 size_t star_ws_bytes(int n, int batch) {
   return (size_t)8 * n * n * sizeof(cd) * batch + (size_t)2 * (n + 1) * batch * sizeof(int) + 256;
 }
@@ -44,16 +70,14 @@ int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, 
   const Mat mRD{RD, 2 * n, 2 * nn}, mRF{RF, 2 * n, 2 * nn};
   const Mat mRD2{RD + n, 2 * n, 2 * nn}, mRF2{RF + n, 2 * n, 2 * nn};
 
+  long long g = (nn * batch + 255) / 256;
+  if (g > 131072) g = 131072;
+  star_prep_kernel<<<dim3((unsigned)g), 256, 0, s>>>(SA, sA, SB, sB, n, batch, D, F, RD, RF, S);
+  KHX_LAUNCH_CHECK();
   // D = I - SB11 SA22 ; F = I - SA22 SB11
-  KHX_TRY(zset_identity(s, mD, n, n, one, batch));
   KHX_TRY(zgemm(s, n, n, n, mone, B11, A22, one, mD, batch));
-  KHX_TRY(zset_identity(s, mF, n, n, one, batch));
   KHX_TRY(zgemm(s, n, n, n, mone, A22, B11, one, mF, batch));
   // [X1 | X2] = D^-1 [SB11 | SB12] ; [Y1 | Y2] = F^-1 [SA21 | SA22]
-  KHX_TRY(zcopy(s, mRD, B11, n, n, batch));
-  KHX_TRY(zcopy(s, mRD2, B12, n, n, batch));
-  KHX_TRY(zcopy(s, mRF, A21, n, n, batch));
-  KHX_TRY(zcopy(s, mRF2, A22, n, n, batch));
   if (gj) {  // (D, F and the right-hand sides follow each other)
     KHX_TRY(zgesv_ws(s, n, 2 * n, mD, mRD, 2 * batch, perm, infos));
   } else {
@@ -62,7 +86,6 @@ int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, 
   }
   // S11 = SA11 + (SA12 X1) SA21
   KHX_TRY(zgemm(s, n, n, n, one, A12, mRD, zero, mT, batch));
-  KHX_TRY(zcopy(s, S11, A11, n, n, batch));
   KHX_TRY(zgemm(s, n, n, n, one, mT, A21, one, S11, batch));
   // S12 = SA12 X2
   KHX_TRY(zgemm(s, n, n, n, one, A12, mRD2, zero, S12, batch));
@@ -70,7 +93,6 @@ int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, 
   KHX_TRY(zgemm(s, n, n, n, one, B21, mRF, zero, S21, batch));
   // S22 = SB22 + (SB21 Y2) SB12
   KHX_TRY(zgemm(s, n, n, n, one, B21, mRF2, zero, mT, batch));
-  KHX_TRY(zcopy(s, S22, B22, n, n, batch));
   KHX_TRY(zgemm(s, n, n, n, one, mT, B12, one, S22, batch));
   if (info) {
     star_info_kernel<<<dim3((batch + 255) / 256), 256, 0, s>>>(infos, batch, info);

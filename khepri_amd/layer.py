@@ -63,6 +63,7 @@ class Layer:
         self.expansion = None
         self.W = self.V = self.L = None
         self.S = None
+        self.skind, self.X = "dense", None
         self.IC = None
         self.fields = False
         self.device = None
@@ -154,6 +155,17 @@ class Layer:
     def chain_item(self):
         return (self.skind, self.X if self.skind == "prop" else self.S)
 
+    def structure(self):
+        """("identity", None) for a half space of the gap medium, ("prop", X) for
+        a uniform layer of it (X its propagation factors), else ("dense", S):
+        what a star product with this layer amounts to."""
+        if np.isscalar(self.epsilon) and complex(self.epsilon) == 1:
+            if self.formulation in (Formulation.HALF_SPACE_INC, Formulation.HALF_SPACE_TRN):
+                return ("identity", None)
+            if self.formulation == Formulation.UNIFORM and self.X is not None:
+                return ("prop", self.X)
+        return ("dense", self.S)
+
     @staticmethod
     def solve_batch_many(layers, kp, wl, rt_only=False, plan=None):
         """solve_batch for several layers of one expansion.  When all their
@@ -236,6 +248,8 @@ class Layer:
             self.C = C
             self.IC = IC if modes else None
         elif self.formulation == Formulation.UNIFORM:
+            if gap_medium:   # the dense S below is [[0, X], [X, 0]]: stack_layers folds X into a neighbour
+                self.X = ops.propagation(kx, ky, (k0 * self.depth).contiguous())
             # 1 / eps as the reference's P = (1/er) [...] (khepri/alternative.py:138):
             # ZeroDivisionError for a Python zero, inf (non-finite R, T) for a numpy one
             inv = 1 / self.epsilon
@@ -287,6 +301,20 @@ def scattering_identity(B, n, device):
     return S
 
 
+def _stack_forward(layers, ws, infos):
+    """Total S-matrix from each layer's structure; None when no layer is dense."""
+    from . import chain
+    seq = chain.dense_sequence([ly.structure() if isinstance(ly, Layer) else ("dense", ly.S) for ly in layers])
+    if len(layers) < 2 or isinstance(seq, tuple) or not seq:
+        return None
+    Stot = seq[0]
+    for S in seq[1:]:
+        Stot, info = ops.redheffer(Stot, S, ws=ws, gj=True)
+        if infos is not None:
+            infos.append(info)
+    return Stot
+
+
 def stack_layers(pw, layers, mask, reverse=True, ws=None, infos=None):
     """Forward chain S_I * S_0 * S_1 * ... (copies kept where mask) and the
     reverse chain (khepri/layer.py:35-60).
@@ -295,8 +323,16 @@ def stack_layers(pw, layers, mask, reverse=True, ws=None, infos=None):
     formed.  The reverse chain is only needed for fields (``reverse=False``
     skips it and returns None for it).  ``infos``, when a list, receives the
     device status word of every star product (first zero pivot of D or F,
-    where the reference's numpy solve raises LinAlgError).
+    where the reference's numpy solve raises LinAlgError).  Without fields
+    and inner copies, layers of the gap medium are not multiplied: its half
+    spaces are the identity, its uniform layers diagonal scalings of a
+    neighbour (a third of the star products of a typical stack are left).
     """
+    if not reverse and not any(mask[1:-1]):
+        Stot = _stack_forward(layers, ws, infos)
+        if Stot is not None:
+            return [layers[0].S if mask[0] else None, *[None] * (len(layers) - 2), Stot if mask[-1] else None], \
+                None, Stot
     Stot = layers[0].S
     Sls = [Stot if mask[0] else None]
     for keep, layer in zip(mask[1:], layers[1:]):
