@@ -200,7 +200,7 @@ int khx_patterned_layer_cached(const double* C, const double* IC, int per_item, 
  * khx_layer_smatrix: S (batch, 2, 2, n, n), one number of doublings for the
  *   whole batch.  info[b]: 1 a non-finite entry in P Q (numpy's eig raises),
  *   -1 a solve met an exact zero pivot, else 0.                            */
-#define KHX_LAYER_THETA 2.75
+#define KHX_LAYER_THETA 4.0
 int khx_layer_scale(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
                     int batch, const double* k0d, double* est, void* stream);
 size_t khx_layer_smatrix_ws_bytes(int n, int batch, int doublings);

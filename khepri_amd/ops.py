@@ -327,9 +327,9 @@ def eig(A, overwrite_a=False):
 
 
 # The slice of a layer may be this thick (|k0 d sqrt(eigenvalue)| / 2): up to
-# here the [13/13] approximant of khx_layer_smatrix is exact to FP64 rounding
+# here the [17/17] approximant of khx_layer_smatrix is exact to FP64 rounding
 # (khx.h: KHX_LAYER_THETA).
-LAYER_THETA = 2.75
+LAYER_THETA = 4.0
 # Layers that need more doublings go through the eigensolver, whose work does
 # not grow with the depth: each doubling is 37 n^3 operations.
 LAYER_MAX_DOUBLINGS = 12
