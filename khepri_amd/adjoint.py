@@ -192,7 +192,7 @@ def _gradient_chunk(cl, names, wrt, g, N, kp, wl, te, tm, wR, wT, eta_rel, reduc
         raise ValueError("the device has no scattering layer")
     Ps = [fwd[seq[0]][1]]
     for nm in seq[1:]:
-        P, info = ops.redheffer(Ps[-1], fwd[nm][1], gj=True)
+        P, info = ops.redheffer(Ps[-1], fwd[nm][1])
         ops.raise_on_info(info, "star product", lu=True)
         Ps.append(P)
     Stot = Ps[-1]

@@ -45,9 +45,10 @@ size_t star_ws_bytes(int n, int batch) {
 
 // gj: both systems in one batch through the two-launch Gauss-Jordan
 // (zgesv_ws; D and F are well conditioned for passive layers).  The chains that
-// fields are read from keep the LU: the mode amplitudes inside a layer are
-// differences of terms as large as e^{lambda d}, and carry every rounding of the
-// chain magnified as much.
+// fields or gradients are read from keep the LU: the mode amplitudes inside a
+// layer are differences of terms as large as e^{lambda d}, the eigenvector
+// adjoint divides by mode differences, and both carry every rounding of the chain
+// magnified as much.
 int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, int n, int batch, cd* S,
          int* info, void* wsv, bool gj) {
   if (batch <= 0) return 0;
@@ -110,7 +111,7 @@ int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, 
 //   [B11bar | B12bar] += D^-H [X1bar | X2bar], Dbar = -D^-H [X1bar | X2bar] [X1 | X2]^H,
 //   and D = I - B11 A22, F = I - A22 B11 pass Dbar, Fbar on to B11 and A22.
 size_t star_bwd_ws_bytes(int n, int batch) {
-  return (size_t)16 * n * n * sizeof(cd) * batch + (size_t)(4 + 2 * n) * batch * sizeof(int) + 256;
+  return (size_t)16 * n * n * sizeof(cd) * batch + (size_t)4 * batch * sizeof(int) + 256;
 }
 
 int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, int n, int batch, const cd* Sbar,
@@ -137,7 +138,6 @@ int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long 
   cd* T1 = take(1);
   cd* T2 = take(1);
   int* infos = reinterpret_cast<int*>(w);
-  int* perm = infos + 4 * (long long)batch;
   auto blk = [&](const cd* base, long long str, int q) { return Mat{const_cast<cd*>(base) + q * nn, n, str}; };
   const Mat A11 = blk(SA, sA, 0), A12 = blk(SA, sA, 1), A21 = blk(SA, sA, 2), A22 = blk(SA, sA, 3);
   const Mat B11 = blk(SB, sB, 0), B12 = blk(SB, sB, 1), B21 = blk(SB, sB, 2), B22 = blk(SB, sB, 3);
@@ -161,7 +161,8 @@ int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long 
   KHX_TRY(zcopy(s, mX2, B12, n, n, batch));
   KHX_TRY(zcopy(s, mRF, A21, n, n, batch));
   KHX_TRY(zcopy(s, mY2, A22, n, n, batch));
-  KHX_TRY(zgesv_ws(s, n, 2 * n, mD, mRD, 2 * batch, perm, infos));
+  KHX_TRY(zgesv(s, n, 2 * n, mD, mRD, batch, infos));
+  KHX_TRY(zgesv(s, n, 2 * n, mF, mRF, batch, infos + batch));
 
   // S11 = A11 + A12 X1 A21, S12 = A12 X2
   KHX_TRY(zcopy(s, a11, G11, n, n, batch));
@@ -184,12 +185,12 @@ int star_bwd(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long 
   KHX_TRY(zgemm(s, n, n, n, one, B21, mY2, zero, mT1, batch));
   KHX_TRY(zgemm_op(s, 2, 0, n, n, n, one, mT1, G22, zero, b12, batch));
   // [X1 | X2] = D^-1 [B11 | B12]
-  KHX_TRY(zgesv_ws(s, n, 2 * n, mDH, mZX, batch, perm, infos + 2 * batch));
+  KHX_TRY(zgesv(s, n, 2 * n, mDH, mZX, batch, infos + 2 * batch));
   KHX_TRY(zcopy(s, b11, mZX, n, n, batch));
   KHX_TRY(zaxpby(s, b12, one, b12, one, mZX2, n, n, batch));
   KHX_TRY(zgemm_op(s, 0, 2, n, n, 2 * n, mone, mZX, mRD, zero, mDb, batch));
   // [Y1 | Y2] = F^-1 [A21 | A22]
-  KHX_TRY(zgesv_ws(s, n, 2 * n, mFH, mZY, batch, perm, infos + 3 * batch));
+  KHX_TRY(zgesv(s, n, 2 * n, mFH, mZY, batch, infos + 3 * batch));
   KHX_TRY(zaxpby(s, a21, one, a21, one, mZY, n, n, batch));
   KHX_TRY(zcopy(s, a22, mZY2, n, n, batch));
   KHX_TRY(zgemm_op(s, 0, 2, n, n, 2 * n, mone, mZY, mRF, zero, mFb, batch));
