@@ -37,7 +37,7 @@ from .layer import plan_layers
 
 
 def _same_plan(a, b):
-    return a.keys() == b.keys() and all((a[k] == b[k]).all() for k in a)
+    return a.keys() == b.keys() and all((a[k].counts == b[k].counts).all() for k in a)
 
 
 class _Captured:

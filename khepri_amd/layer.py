@@ -173,7 +173,7 @@ class Layer:
         patterned layers are solved together in one fused call so that they
         share the GPU (a single layer's small batch leaves most CUs idle); the
         bound also keeps the fused workspace within one round's worth of
-        items.  plan: {id(layer): doublings per source}, from plan_layers.
+        items.  plan: {id(layer): Doublings of its sources}, from plan_layers.
         Everything else as solve_batch."""
         plan = plan or {}
         pat = [ly for ly in layers if getattr(ly, "patterned", False)]
@@ -192,7 +192,7 @@ class Layer:
         known = [plan.get(id(ly)) for ly in pat]
         res = ops.patterned_layers_fused([m[0] for m in mats], [m[1] for m in mats], kx, ky,
                                          [(k0 * ly.depth).contiguous() for ly in pat], modes=modes,
-                                         doublings=None if any(d is None for d in known) else np.concatenate(known))
+                                         doublings=None if any(d is None for d in known) else ops.Doublings.cat(known))
         for ly, (C, IC), (S, (W, V, L), info) in zip(pat, mats, res):
             ly.device = dev
             ly.skind, ly.X = "dense", None
@@ -271,7 +271,7 @@ _PLAN_SOURCES = 16384
 
 
 def plan_layers(layers, kp, wl):
-    """{id(layer): doublings per source} for the layers of a stack whose
+    """{id(layer): Doublings of its sources} for the layers of a stack whose
     S-matrices are formed without modes, over all sources of a solve: one
     estimate launch per layer and slice of sources, one host synchronisation
     at the end (none between the chunks of the solve)."""
@@ -289,7 +289,8 @@ def plan_layers(layers, kp, wl):
         return {}
     sizes = [len(v) for v in est.values()]
     counts = ops.doublings_of(torch.cat(list(est.values())))
-    return dict(zip(est, np.split(counts, np.cumsum(sizes)[:-1])))
+    ends = np.cumsum([0, *sizes])
+    return {key: counts[a:b] for key, a, b in zip(est, ends, ends[1:])}
 
 
 def scattering_identity(B, n, device):

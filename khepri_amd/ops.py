@@ -353,13 +353,44 @@ def layer_scale(C, IC, kx, ky, k0d):
     return est
 
 
+class Doublings:
+    """Doubling counts of a batch of layers (counts: host int array; -1: through
+    the eigensolver).  Slices and concatenations share one memo of the device
+    index tensors of the items of each count, so a call repeated under stream
+    capture copies nothing from the host."""
+
+    def __init__(self, counts, memo=None):
+        self.counts = counts
+        self._memo = {} if memo is None else memo
+
+    def __len__(self):
+        return len(self.counts)
+
+    def __getitem__(self, sl):
+        return Doublings(self.counts[sl], self._memo)
+
+    @staticmethod
+    def cat(parts):
+        return parts[0] if len(parts) == 1 else Doublings(np.concatenate([p.counts for p in parts]), parts[0]._memo)
+
+    def groups(self, device):
+        """[(count, indices of its items on the device, or None for all of them)]"""
+        values = np.unique(self.counts)
+        if len(values) == 1:
+            return [(int(values[0]), None)]
+        key = (str(device), self.counts.tobytes())
+        if key not in self._memo:
+            self._memo[key] = [(int(v), torch.as_tensor(np.nonzero(self.counts == v)[0], device=device))
+                               for v in values]
+        return self._memo[key]
+
+
 def doublings_of(est):
-    """Doublings per item (int array on the host) for layer_scale's estimates;
-    -1 for the items that go through the eigensolver.  A host synchronisation."""
+    """The Doublings of layer_scale's estimates.  A host synchronisation."""
     with np.errstate(all="ignore"):
         e = est.cpu().numpy() / LAYER_THETA
         s = np.where(e > 1.0, np.ceil(np.log2(np.where(e > 1.0, e, 1.0))), 0.0)   # NaN: 0, flagged by the kernel
-    return np.where(s > LAYER_MAX_DOUBLINGS, -1, s).astype(np.int64)
+    return Doublings(np.where(s > LAYER_MAX_DOUBLINGS, -1, s).astype(np.int64))
 
 
 def _layer_smatrix(C, IC, kx, ky, k0d, doublings, S, info):
@@ -372,31 +403,29 @@ def _layer_smatrix(C, IC, kx, ky, k0d, doublings, S, info):
 
 def layer_smatrix(C, IC, kx, ky, k0d, doublings):
     """(S (B, 2, 2, n, n), status words) of a patterned layer without its
-    modes; doublings: int array (B,) as doublings_of gives it.  The items of
-    one count are solved together, so an item's result does not depend on the
-    batch it comes in."""
+    modes; doublings: the items' Doublings.  The items of one count
+    are solved together, so an item's result does not depend on the batch it
+    comes in."""
     B, N = kx.shape
     n = 2 * N
     dev = kx.device
     S = torch.empty((B, 2, 2, n, n), dtype=CDT, device=dev)
     info = torch.empty(B, dtype=torch.int32, device=dev)
-    counts = np.unique(doublings)
-    for s in counts:
-        if len(counts) == 1:
-            args, Sg, ig = (C, IC, kx, ky, k0d), S, info
+    for s, idx in doublings.groups(dev):
+        if idx is None:
+            b, args = B, (C, IC, kx, ky, k0d)
         else:
-            idx = torch.as_tensor(np.nonzero(doublings == s)[0], device=dev)
-            Cg, ICg = (C[idx], IC[idx]) if C.dim() == 3 else (C, IC)
-            args = (Cg, ICg, kx[idx], ky[idx], k0d[idx])
-            Sg = torch.empty((len(idx), 2, 2, n, n), dtype=CDT, device=dev)
-            ig = torch.empty(len(idx), dtype=torch.int32, device=dev)
+            b = len(idx)
+            args = (*((C[idx], IC[idx]) if C.dim() == 3 else (C, IC)), kx[idx], ky[idx], k0d[idx])
+        Sg = S if idx is None else torch.empty((b, 2, 2, n, n), dtype=CDT, device=dev)
+        ig = info if idx is None else torch.empty(b, dtype=torch.int32, device=dev)
         if s < 0:
             Sm, _, im = _modal_layer(*args)
             Sg.copy_(Sm)
             ig.copy_(im)
         else:
-            _layer_smatrix(*args, int(s), Sg, ig)
-        if len(counts) > 1:
+            _layer_smatrix(*args, s, Sg, ig)
+        if idx is not None:
             S[idx] = Sg
             info[idx] = ig
     return S, info
@@ -409,7 +438,7 @@ def patterned_layer(C, IC, kx, ky, k0d, modes=False, ws=None, cache=None, doubli
     patterned_layer_bwd (khx_patterned_layer_cached).
 
     Without modes and cache the S-matrix is formed directly
-    (khx_layer_smatrix); doublings: the items' counts if the caller has them
+    (khx_layer_smatrix); doublings: the items' Doublings if the caller has them
     (doublings_of(layer_scale(...))), else they are determined here, with a
     host synchronisation -- which a stream capture does not allow, so a
     captured call without them goes through the eigensolver."""
@@ -540,7 +569,7 @@ def analytic_layer(kind, kx, ky, eps, k0d=None, modes=False):
 def redheffer(SA, SB, out=None, ws=None, gj=False):
     """SA * SB, with its status words; gj: the two solves through
     khx_zgesv_ws's Gauss-Jordan in one batch -- for chains that only R, T or S
-    are read from (a chain that fields are read from keeps the LU)."""
+    are read from (a chain that fields or gradients are read from keeps the LU)."""
     lib = _lib.load()
     ab = SA.dim() == 4
     bb = SB.dim() == 4

@@ -70,7 +70,7 @@ def test_items_of_different_counts_match_single_solves(gpu):
     kx, ky = ops.kvectors(lys[0].expansion.g_device(gpu), kp, wls)
     k0d = 2 * np.pi / wls * torch.as_tensor(depths, device=gpu)
     counts = ops.doublings_of(ops.layer_scale(C, IC, kx, ky, k0d))
-    assert len(set(counts.tolist())) >= 3
+    assert len(set(counts.counts.tolist())) >= 3
     S, _, info = ops.patterned_layer(C, IC, kx, ky, k0d)
     assert (info.cpu().numpy() == 0).all()
     for k, ly in enumerate(lys):
@@ -117,10 +117,11 @@ def test_graph_recaptures_when_the_counts_change(gpu):
     cl = crystal()
     cl.set_source(np.array([1.9, 2.0]), 1.0, 0.0)
     g = SolveGraph(cl)
-    before = {k: v.copy() for k, v in g.plan.items()}
-    kp = np.array([[12.0, 9.0], [13.0, 8.0]])      # far evanescent: larger |K|
+    before = {k: v.counts.copy() for k, v in g.plan.items()}
+    kp = np.array([[0.3, 0.2], [90.0, 80.0]])      # the second far evanescent: the counts differ in the batch
     g.update_sources(np.array([1.9, 2.0]), 1.0, 0.0, kp=kp)
-    assert any((before[k] != g.plan[k]).any() for k in before)
+    assert any((before[k] != g.plan[k].counts).any() for k in before)
+    assert any(len(set(d.counts.tolist())) == 2 for d in g.plan.values())
     for _ in range(2):
         R, T = g.replay()
         ref = crystal()
@@ -137,4 +138,4 @@ def test_doubling_rule():
     t = ops.LAYER_THETA
     est = torch.tensor([0.0, t, t * 1.001, 2 * t, 2.001 * t, t * 2.0 ** 12, t * 2.0 ** 12 * 1.001, float("nan"),
                         float("inf")], dtype=torch.float64)
-    assert ops.doublings_of(est).tolist() == [0, 0, 1, 1, 2, 12, -1, 0, -1]
+    assert ops.doublings_of(est).counts.tolist() == [0, 0, 1, 1, 2, 12, -1, 0, -1]
