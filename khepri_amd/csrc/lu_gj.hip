@@ -1,4 +1,4 @@
-// Batched complex solve A X = B in two launches: blocked Gauss-Jordan with
+// Batched complex solve A X = B in few launches: blocked Gauss-Jordan with
 // partial pivoting in product form, for orders up to GJ_MAX_N.
 //
 // The columns of A are taken in panels of 16.  Eliminating a panel's columns
@@ -10,24 +10,26 @@
 // each column was eliminated with: rows are never moved, so nothing is
 // interchanged, and X[k] is row perm[k] of the transformed B.
 //
-// gj_factor_kernel: one workgroup per system, a wavefront per 64 rows.  A
-//   panel's columns are loaded into MFMA accumulators, all earlier panels are
-//   applied to them (left-looking: A is read and written once), and the panel
-//   is eliminated in registers, one row per lane: a pivot step is one integer
-//   maximum over the lanes (DPP), one LDS exchange of the pivot row and one
-//   barrier.
-// gj_solve_kernel: one workgroup per system and strip of 16 CB columns of B.
-//   The strip stays in MFMA accumulators from its load to its store while the
-//   n / 16 panels pass by: 8 n^2 operations per column on the matrix cores with
-//   B moved once; the 16 pivot rows of a panel go through LDS, G comes from L2
-//   (the strips of one system run on one XCD).
+// gj_factor_kernel: 64, 128 or all columns in one launch, one workgroup per
+//   system, a wavefront per 48 or 64 rows.  A panel's columns are loaded into MFMA
+//   accumulators, the launch's earlier panels are applied to them (left-looking:
+//   A is read and written once), and the panel is eliminated in registers, one
+//   row per lane: a pivot step is one integer maximum over the lanes (DPP), one
+//   LDS exchange of the pivot row and one barrier.
+// gj_strips_kernel: one workgroup per system and strip of 16 CB columns, of B or
+//   of the columns of A still to be factored.  The strip stays in MFMA
+//   accumulators from its load to its store while the panels pass by: 8 n^2
+//   operations per column on the matrix cores with B moved once; the 16 pivot
+//   rows of a panel go through LDS, G comes from L2 (the strips of one system run
+//   on one XCD).
 // The multi-launch LU (lu_blocked.hip) needs 11 panel launches, as many trailing
 // updates and 22 leaf launches for n = 162 and moves the trailing matrix once per
 // panel.  Measured, LU -> here, ms: n = 50 (50 right-hand sides) 2 systems 0.28 ->
-// 0.08, 4 096 systems 4.4 -> 0.43; n = 162 (162) 2 048 systems 7.0 -> 3.7; n = 338
-// (338) 512 systems 11.1 -> 7.2.  The solve runs at about 70 % of the FP64 matrix
-// rate; the factorization is bound by the latency of its pivot steps (about 1 us:
-// maximum, LDS exchange, barrier, reciprocal).
+// 0.08, 4 096 systems 4.4 -> 0.42; n = 162 (162) 2 048 systems 7.0 -> 3.6; n = 338
+// (338) 512 systems 11.1 -> 7.1, 2 systems (1.5 when one launch factored all
+// columns) 0.89.  The solve runs at about 70 % of the FP64 matrix rate; the
+// factorization is bound by the latency of its pivot steps (about 1 us: maximum,
+// LDS exchange, barrier, reciprocal).
 // Error: forward error as an LU's; the residual of an ill-conditioned system can
 // be larger (Gauss-Jordan is not row-wise backward stable), so it serves the
 // systems that are well conditioned by construction.
@@ -155,22 +157,22 @@ __device__ __forceinline__ void multiply(Strip<RB, CB>& x, const Frag<RB>& f, co
     }
 }
 
-// panels 0 .. panels - 1 in order; Y: two buffers of 17 x (16 CB + 1); nbl:
-// columns of the last panel
+// panels j0 .. j1 - 1 in order; Y: two buffers of 17 x (16 CB + 1); nbl: columns
+// of panel j1 - 1
 template <int RB, int CB>
-__device__ __forceinline__ void apply_panels(Strip<RB, CB>& x, const cd* __restrict__ a, int lda, int n, int panels,
+__device__ __forceinline__ void apply_panels(Strip<RB, CB>& x, const cd* __restrict__ a, int lda, int n, int j0, int j1,
                                              int nbl, lcd* Y, int row0, int li, int lk) {
   constexpr int YC = 16 * CB + 1;
-  if (panels <= 0) return;
+  if (j0 >= j1) return;
   const int left = n - row0, blocks = left <= 0 ? 0 : (left + 15) / 16;
   unsigned roff[RB];
 #pragma unroll
   for (int t = 0; t < RB; ++t) roff[t] = (unsigned)(min(row0 + t * 16 + li, n - 1) * lda);
   Frag<RB> f0, f1;
-  fetch(f0, a, roff, 4 * lk, n - 1);
-  for (int j = 0; j < panels; ++j) {
+  fetch(f0, a, roff, j0 * NB + 4 * lk, n - 1);
+  for (int j = j0; j < j1; ++j) {
     lcd* y = Y + (j & 1) * (NB + 1) * YC;
-    if (nbl < NB && j == panels - 1)  // the rows that a narrower last panel does not have
+    if (nbl < NB && j == j1 - 1)  // the rows that a narrower last panel does not have
       for (int e = threadIdx.x; e < (NB - nbl) * YC; e += blockDim.x) y[nbl * YC + e] = lcd{0.0, 0.0};
     take_pivot_rows(x, j * NB, y, li);
     fetch(f1, a, roff, j * NB + 4 * lk + 2, n - 1);
@@ -189,10 +191,11 @@ struct Candidate {
 };
 constexpr int GJ_MAX_WAVES = 8;
 
-// Workgroups of ceil(n / (16 RB)) wavefronts; in the elimination lane l of
-// wavefront w owns row 16 RB w + l (l < 16 RB).
+// Columns c0 .. c1 - 1 (c0 a multiple of 16), to which the panels before c0 have
+// been applied.  Workgroups of ceil(n / (16 RB)) wavefronts; in the elimination
+// lane l of wavefront w owns row 16 RB w + l (l < 16 RB).
 template <int RB>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3 : 2))) void gj_factor_kernel(int n, cd* A, int lda, long long sA, int* perm, int* info) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3 : 2))) void gj_factor_kernel(int n, int c0, int c1, cd* A, int lda, long long sA, int* perm, int* info) {
   extern __shared__ lcd sm[];
   const int nw = blockDim.x >> 6;
   lcd* stage = sm;                                                         // nw x 16 x YS, wavefront-private
@@ -207,11 +210,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3
   const int row0 = wave * 16 * RB;
   const int row = lane < 16 * RB ? row0 + lane : n;  // the row this lane eliminates
   int first_zero = 0;
-  bool open = row < n;
   for (int e = tid; e < 16 * RB * nw; e += blockDim.x) ord[e] = 1 << 30;
   if (tid < GJ_MAX_WAVES) keys[tid] = make_int4(-2, 0, -2, 0);
   __syncthreads();
-  for (int k0 = 0; k0 < n; k0 += NB) {
+  for (int k = tid; k < c0; k += blockDim.x) ord[perm[item * n + k]] = k;
+  __syncthreads();
+  bool open = row < n && ord[min(row, n - 1)] == 1 << 30;
+  for (int k0 = c0; k0 < c1; k0 += NB) {
     const int nb = min(NB, n - k0);
     cd x[NB];
     {
@@ -229,7 +234,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3
           st.im[t][0][r] = v.y;
           st.slot[t][r] = ord[gr];
         }
-      apply_panels(st, a, lda, n, k0 / NB, NB, Y, row0, li, lk);
+      apply_panels(st, a, lda, n, c0 / NB, k0 / NB, NB, Y, row0, li, lk);
       // accumulators -> one row per lane, 16 rows at a time through the
       // wavefront's own LDS
       lcd* sp = stage + wave * 16 * YS;
@@ -256,33 +261,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3
     // key: the high word of |re| + |im| orders the candidates to 2^-20; rows
     // already used have -1
     int key = open ? __double2hiint(cabs1(x[0])) & 0x7fffffff : -1;
+    cd rc = recip_pivot(x[0]);
+    int best = wave_max_int(key);
 #pragma unroll 1
     for (int jj = 0; jj < nb; ++jj) {
       const int buf = (jj & 1) * GJ_MAX_WAVES;
-      const cd rc = recip_pivot(x[0]);
-      const int best = wave_max_int(key);
       const int src = __ffsll((unsigned long long)__ballot(key == best)) - 1;
       if (lane == src) {
         Candidate& c = cand[buf + wave];
+        reinterpret_cast<int2*>(keys)[buf + wave] = make_int2(best, row);
 #pragma unroll
         for (int q = 0; q < NB; ++q) c.row[q] = lcd{x[q].x, x[q].y};
         c.recip = lcd{rc.x, rc.y};
-        reinterpret_cast<int2*>(keys)[buf + wave] = make_int2(best, row);
       }
       __syncthreads();
-      int4 kq[GJ_MAX_WAVES / 2];
+      int w = 0, kbest = best, prow = row0 + src;
+      if (nw > 1) {
+        int4 kq[GJ_MAX_WAVES / 2];
 #pragma unroll
-      for (int q = 0; q < GJ_MAX_WAVES / 2; ++q) kq[q] = keys[buf / 2 + q];
-      int w = 0, kbest = kq[0].x, prow = kq[0].y;
+        for (int q = 0; q < GJ_MAX_WAVES / 2; ++q) kq[q] = keys[buf / 2 + q];
+        kbest = kq[0].x;
+        prow = kq[0].y;
 #pragma unroll
-      for (int q = 1; q < GJ_MAX_WAVES; ++q) {
-        const int k = q & 1 ? kq[q / 2].z : kq[q / 2].x, r = q & 1 ? kq[q / 2].w : kq[q / 2].y;
-        const bool more = k > kbest;
-        w = more ? q : w;
-        prow = more ? r : prow;
-        kbest = more ? k : kbest;
+        for (int q = 1; q < GJ_MAX_WAVES; ++q) {
+          const int k = q & 1 ? kq[q / 2].z : kq[q / 2].x, r = q & 1 ? kq[q / 2].w : kq[q / 2].y;
+          const bool more = k > kbest;
+          w = more ? q : w;
+          prow = more ? r : prow;
+          kbest = more ? k : kbest;
+        }
+        w = __builtin_amdgcn_readfirstlane(w);
       }
-      w = __builtin_amdgcn_readfirstlane(w);
       const Candidate& c = cand[buf + w];
       const lcd rp = c.recip;
       lcd pa[8], pb[7];
@@ -298,22 +307,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3
 #pragma unroll
         for (int q = 0; q < NB; ++q) x[q] = mkc(0.0, 0.0);
       }
+      // the next column first: its pivot search and reciprocals run beside the
+      // other columns' updates
+      x[0] = fmsc(x[1], m, mkc(pa[0].x, pa[0].y));
+      key = open ? __double2hiint(cabs1(x[0])) & 0x7fffffff : -1;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        x[q] = fmsc(x[q + 1], m, mkc(pa[q].x, pa[q].y));
-        pb[q] = c.row[q + 9];
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int q = 0; q < 7; ++q) pb[q] = c.row[q + 9];
+      rc = recip_pivot(x[0]);
+      best = wave_max_int(key);
 #pragma unroll
-      for (int q = 4; q < 8; ++q) {
-        x[q] = fmsc(x[q + 1], m, mkc(pa[q].x, pa[q].y));
-        if (q < 7) pb[q] = c.row[q + 9];
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int q = 1; q < 8; ++q) x[q] = fmsc(x[q + 1], m, mkc(pa[q].x, pa[q].y));
 #pragma unroll
       for (int q = 8; q < NB - 1; ++q) x[q] = fmsc(x[q + 1], m, mkc(pb[q - 8].x, pb[q - 8].y));
       x[NB - 1] = -m;
-      key = open ? __double2hiint(cabs1(x[0])) & 0x7fffffff : -1;
     }
     for (int jj = nb; jj < NB; ++jj) {  // the last panel: rotate on
       const cd t = x[0];
@@ -328,15 +334,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3
     }
     __syncthreads();  // G and ord of this panel are read by the other wavefronts
   }
-  if (row < n) perm[item * n + ord[row]] = row;
-  if (tid == 0 && info) info[item] = first_zero;
+  if (row < n) {
+    const int k = ord[row];
+    if (k >= c0 && k < c1) perm[item * n + k] = row;
+  }
+  if (tid == 0 && info && (c0 == 0 || (first_zero && info[item] == 0))) info[item] = first_zero;
 }
 
 // ------------------------------------------------------------ right-hand sides
-template <int RB, int CB>
-__global__ __launch_bounds__(512) void gj_solve_kernel(int n, int m, const cd* __restrict__ A, int lda, long long sA,
-                                                       cd* B, int ldb, long long sB, const int* __restrict__ perm,
-                                                       int strips, int xcd_remap) {
+// Panels j0 .. j1 - 1 on the strips of B (n x m).  LAST: the rows come out in the
+// order of the unknowns (after the last panel); else they stay where they are.
+template <int RB, int CB, bool LAST>
+__global__ __launch_bounds__(512) void gj_strips_kernel(int n, int m, int j0, int j1, const cd* A, int lda,
+                                                        long long sA, cd* B, int ldb, long long sB,
+                                                        const int* __restrict__ perm, int strips, int xcd_remap) {
   extern __shared__ lcd sm[];
   constexpr int YC = 16 * CB + 1;
   lcd* Y = sm;                                               // 2 x 17 x YC
@@ -354,12 +365,10 @@ __global__ __launch_bounds__(512) void gj_solve_kernel(int n, int m, const cd* _
   const int li = lane & 15, lk = lane >> 4;
   const int row0 = wave * 16 * RB;
   const int rows = (blockDim.x >> 6) * 16 * RB;
-  for (int k = tid; k < rows; k += blockDim.x)
-    if (k < n)
-      ord[perm[item * n + k]] = k;
-    else
-      ord[k] = 1 << 30;
-  const int panels = (n + NB - 1) / NB, nbl = n - (panels - 1) * NB;
+  const int k0 = j0 * NB, k1 = min(n, j1 * NB);
+  for (int k = tid; k < rows; k += blockDim.x) ord[k] = 1 << 30;
+  __syncthreads();
+  for (int k = k0 + tid; k < k1; k += blockDim.x) ord[perm[item * n + k]] = k;
   Strip<RB, CB> x;
 #pragma unroll
   for (int t = 0; t < RB; ++t)
@@ -377,14 +386,14 @@ __global__ __launch_bounds__(512) void gj_solve_kernel(int n, int m, const cd* _
   for (int t = 0; t < RB; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) x.slot[t][r] = ord[row0 + t * 16 + lk + 4 * r];
-  apply_panels(x, a, lda, n, panels, nbl, Y, row0, li, lk);
+  apply_panels(x, a, lda, n, j0, j1, k1 - (j1 - 1) * NB, Y, row0, li, lk);
 #pragma unroll
   for (int t = 0; t < RB; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int gr = row0 + t * 16 + lk + 4 * r;
       if (gr >= n) continue;
-      const int k = x.slot[t][r];
+      const int k = LAST ? x.slot[t][r] : gr;
 #pragma unroll
       for (int u = 0; u < CB; ++u) {
         const int gc = col0 + u * 16 + li;
@@ -393,26 +402,46 @@ __global__ __launch_bounds__(512) void gj_solve_kernel(int n, int m, const cd* _
     }
 }
 
-template <int RB, int CB>
-int launch_solve(hipStream_t s, int n, int m, Mat A, Mat B, int batch, const int* perm) {
+template <int RB, int CB, bool LAST>
+int launch_strips(hipStream_t s, int n, int m, int j0, int j1, Mat A, Mat B, int batch, const int* perm) {
   const int th = 64 * ((n + 16 * RB - 1) / (16 * RB));
   const int strips = (m + 16 * CB - 1) / (16 * CB);
   const long long blocks = (long long)strips * batch;
   KHX_REQUIRE(blocks < (1ll << 31), "zgesv: grid too large");
   const size_t lds = (size_t)2 * (NB + 1) * (16 * CB + 1) * sizeof(lcd) + (size_t)(th / 64) * 16 * RB * sizeof(int);
-  gj_solve_kernel<RB, CB><<<dim3((unsigned)blocks), dim3(th), lds, s>>>(n, m, A.p, A.ld, A.stride, B.p, B.ld,
-                                                                       B.stride, perm, strips, blocks % 8 == 0 ? 1 : 0);
+  gj_strips_kernel<RB, CB, LAST><<<dim3((unsigned)blocks), dim3(th), lds, s>>>(
+      n, m, j0, j1, A.p, A.ld, A.stride, B.p, B.ld, B.stride, perm, strips, blocks % 8 == 0 ? 1 : 0);
   KHX_LAUNCH_CHECK();
   return 0;
 }
 
+// Rows per wavefront: as few as give four wavefronts.  Strips of 32 columns halve
+// the traffic of G (n = 338, 512 systems: 3.4 against 3.8 ms); narrower ones
+// spread a small batch over more CUs.
+template <bool LAST>
+int strips_sized(hipStream_t s, int n, int m, int j0, int j1, Mat A, Mat B, int batch, const int* perm) {
+  const int rb = n <= 64 ? 1 : n <= 128 ? 2 : n <= 192 ? 3 : n <= 256 ? 4 : n <= 384 ? 3 : 4;
+  const int nw = (n + 16 * rb - 1) / (16 * rb);
+  const bool wide = m > 16 && (long long)batch * ((m + 31) / 32) * nw >= 2048;
+  switch (rb * 2 + (wide ? 1 : 0)) {
+    case 2: return launch_strips<1, 1, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+    case 3: return launch_strips<1, 2, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+    case 4: return launch_strips<2, 1, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+    case 5: return launch_strips<2, 2, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+    case 6: return launch_strips<3, 1, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+    case 7: return launch_strips<3, 2, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+    case 8: return launch_strips<4, 1, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+    default: return launch_strips<4, 2, LAST>(s, n, m, j0, j1, A, B, batch, perm);
+  }
+}
+
 template <int RB>
-int launch_factor(hipStream_t s, int n, Mat A, int batch, int* perm, int* info) {
+int launch_factor(hipStream_t s, int n, int c0, int c1, Mat A, int batch, int* perm, int* info) {
   const int nw = (n + 16 * RB - 1) / (16 * RB);
   const size_t lds = (size_t)(nw * 16 + 2 * (NB + 1)) * YS * sizeof(lcd) + 2 * GJ_MAX_WAVES * (sizeof(Candidate) + sizeof(int2)) +
                      (size_t)nw * 16 * RB * sizeof(int);
   KHX_TRY(ensure_dynamic_lds((const void*)gj_factor_kernel<RB>, lds));
-  gj_factor_kernel<RB><<<dim3((unsigned)batch), dim3(64 * nw), lds, s>>>(n, A.p, A.ld, A.stride, perm, info);
+  gj_factor_kernel<RB><<<dim3((unsigned)batch), dim3(64 * nw), lds, s>>>(n, c0, c1, A.p, A.ld, A.stride, perm, info);
   KHX_LAUNCH_CHECK();
   return 0;
 }
@@ -431,30 +460,31 @@ int zgj_solve(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* perm, i
   KHX_REQUIRE((A.stride != 0 && B.stride != 0) || batch == 1, "zgesv: operands cannot be broadcast");
   KHX_REQUIRE((long long)A.ld * n < (1ll << 31), "zgesv: row stride too large");
   ProfScope ps("zgesv_kernel", s);
-  // Rows per wavefront.  Factor: 64 while one or two wavefronts hold the matrix
-  // (fewer barriers per pivot; n = 98, 1 000 systems: 0.33 ms against 0.44 with
-  // 32), 48 where 64 would leave three wavefronts on four SIMDs (n = 162, 2 048:
-  // 1.96 against 2.27 ms).  Solve: as few rows as give four wavefronts.
-  const int rbf = n <= 128 ? 4 : n <= 192 ? 3 : n <= 256 ? 4 : n <= 384 ? 3 : 4;
-  const int rbs = n <= 64 ? 1 : n <= 128 ? 2 : n <= 192 ? 3 : n <= 256 ? 4 : n <= 384 ? 3 : 4;
-  if (rbf == 3)
-    KHX_TRY(launch_factor<3>(s, n, A, batch, perm, info));
-  else
-    KHX_TRY(launch_factor<4>(s, n, A, batch, perm, info));
-  // strips of 32 columns halve the traffic of G (n = 338, 512 systems: 3.4
-  // against 3.8 ms); narrower ones spread a small batch over more CUs
-  const int nw = (n + 16 * rbs - 1) / (16 * rbs);
-  const bool wide = m > 16 && (long long)batch * ((m + 31) / 32) * nw >= 2048;
-  switch (rbs * 2 + (wide ? 1 : 0)) {
-    case 2: return launch_solve<1, 1>(s, n, m, A, B, batch, perm);
-    case 3: return launch_solve<1, 2>(s, n, m, A, B, batch, perm);
-    case 4: return launch_solve<2, 1>(s, n, m, A, B, batch, perm);
-    case 5: return launch_solve<2, 2>(s, n, m, A, B, batch, perm);
-    case 6: return launch_solve<3, 1>(s, n, m, A, B, batch, perm);
-    case 7: return launch_solve<3, 2>(s, n, m, A, B, batch, perm);
-    case 8: return launch_solve<4, 1>(s, n, m, A, B, batch, perm);
-    default: return launch_solve<4, 2>(s, n, m, A, B, batch, perm);
+  // Columns factored by one launch before the others are brought up to date.  One
+  // workgroup per system factors, so few systems leave most of the chip to the
+  // updates' strips, and panels of a launch that reads back little cost little:
+  // 64 columns below 256 systems (n = 338, 16 systems: 1.01 ms against 1.14 with
+  // 128 and 1.82 in one launch; n = 162, 64: 0.37 / 0.38 / 0.40).  Beyond, the CUs
+  // are full either way: 128 columns where G outgrows what a CU's cache keeps
+  // (n = 338, 512 systems: 7.4 / 7.1 / 7.5 ms), all at once up to n = 192 (n =
+  // 162, 1 024: 2.06 / 1.99 / 1.90).
+  const int wb = batch < 256 ? 64 : n > 192 ? 128 : n;
+  // Rows per wavefront of the factorization: 64 while one or two wavefronts hold
+  // the matrix (fewer barriers per pivot; n = 98, 1 000 systems: 0.56 ms against
+  // 0.72 with 48), 48 where 64 would leave three wavefronts on four SIMDs (n =
+  // 162, 2 048: 3.7 against 4.0 ms), 64 again where four or more are needed
+  // (n = 338, 48: 1.48 against 1.53 ms).
+  const int rbf = n > 128 && n <= 192 ? 3 : 4;
+  for (int c0 = 0; c0 < n; c0 += wb) {
+    const int c1 = c0 + wb < n ? c0 + wb : n;
+    if (rbf == 3)
+      KHX_TRY(launch_factor<3>(s, n, c0, c1, A, batch, perm, info));
+    else
+      KHX_TRY(launch_factor<4>(s, n, c0, c1, A, batch, perm, info));
+    if (c1 < n)
+      KHX_TRY(strips_sized<false>(s, n, n - c1, c0 / NB, c1 / NB, A, Mat{A.p + c1, A.ld, A.stride}, batch, perm));
   }
+  return strips_sized<true>(s, n, m, 0, (n + NB - 1) / NB, A, B, batch, perm);
 }
 
 }  // namespace khx

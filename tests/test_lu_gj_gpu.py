@@ -1,4 +1,4 @@
-"""Two-launch Gauss-Jordan solve (khx_zgesv_ws, lu_gj.hip) against numpy, at the
+"""Gauss-Jordan solve (khx_zgesv_ws, lu_gj.hip) against numpy, at the
 orders where its tiling changes: one panel and less (1, 15, 16, 17), the edges of
 the wavefront tilings (64/65, 128/129, 192/193, 256/257, 384/385, 512) and
 beyond them (the LU path), right-hand sides around the 16- and 32-column strips,
@@ -66,3 +66,19 @@ def test_singular_and_nan_items(gpu, n):
     for b in (0, 3):
         ref = np.linalg.solve(A[b], B[b])
         assert np.linalg.norm(X[b] - ref) <= 64e-16 * n * np.linalg.cond(A[b]) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n,m,batch", [(192, 9, 256), (193, 17, 255), (193, 17, 256), (256, 3, 256), (257, 40, 257)])
+def test_columns_in_several_launches(gpu, n, m, batch):
+    """Around the batch and the order from which 64, 128 or all columns are
+    factored by one launch; a zero column in a later launch is reported."""
+    rng = np.random.default_rng(n + batch)
+    A = rng.normal(size=(batch, n, n)) + 1j * rng.normal(size=(batch, n, n))
+    B = rng.normal(size=(batch, n, m)) + 1j * rng.normal(size=(batch, n, m))
+    A[1, :, 150] = 0.0
+    X, info = _solve(A, B, gpu)
+    assert info[1] == 151 and (np.delete(info, 1) == 0).all()
+    for b in (0, batch // 2, batch - 1):
+        ref = np.linalg.solve(A[b], B[b])
+        err = np.linalg.norm(X[b] - ref) / np.linalg.norm(ref)
+        assert err <= 64e-16 * n * np.linalg.cond(A[b]), (b, err)
