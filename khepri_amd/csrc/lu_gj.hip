@@ -10,12 +10,15 @@
 // each column was eliminated with: rows are never moved, so nothing is
 // interchanged, and X[k] is row perm[k] of the transformed B.
 //
-// gj_factor_kernel: 64, 128 or all columns in one launch, one workgroup per
-//   system, a wavefront per 48 or 64 rows.  A panel's columns are loaded into MFMA
-//   accumulators, the launch's earlier panels are applied to them (left-looking:
-//   A is read and written once), and the panel is eliminated in registers, one
-//   row per lane: a pivot step is one integer maximum over the lanes (DPP), one
-//   LDS exchange of the pivot row and one barrier.
+// gj_factor_kernel: 32 columns and more in one launch, one workgroup per system.  A
+//   panel's columns are loaded into MFMA accumulators, the launch's earlier
+//   panels are applied to them (left-looking: A is read and written once), and
+//   the panel is eliminated where it lies, a column per lane of 16 and 16 rows per
+//   four registers.  A pivot step: the rows' keys are made as the values are, the
+//   wavefronts' candidate rows go through LDS as one 16-byte word per lane, the
+//   multipliers come from the column's lane by DPP; one barrier.  (One row per lane
+//   costs 33 LDS words per step and wavefront instead of 3, at 30 to 36 clocks
+//   each: n = 50, 302 systems 0.105 -> 0.087 ms, n = 338, 2 systems 0.88 -> 0.72.)
 // gj_strips_kernel: one workgroup per system and strip of 16 CB columns, of B or
 //   of the columns of A still to be factored.  The strip stays in MFMA
 //   accumulators from its load to its store while the panels pass by: 8 n^2
@@ -25,11 +28,11 @@
 // The multi-launch LU (lu_blocked.hip) needs 11 panel launches, as many trailing
 // updates and 22 leaf launches for n = 162 and moves the trailing matrix once per
 // panel.  Measured, LU -> here, ms: n = 50 (50 right-hand sides) 2 systems 0.28 ->
-// 0.08, 4 096 systems 4.4 -> 0.42; n = 162 (162) 2 048 systems 7.0 -> 3.6; n = 338
-// (338) 512 systems 11.1 -> 7.1, 2 systems (1.5 when one launch factored all
-// columns) 0.89.  The solve runs at about 70 % of the FP64 matrix rate; the
-// factorization is bound by the latency of its pivot steps (about 1 us: maximum,
-// LDS exchange, barrier, reciprocal).
+// 0.055, 4 096 systems 4.4 -> 0.37; n = 162 (162) 2 048 systems 7.0 -> 3.55; n =
+// 338 (338) 512 systems 11.1 -> 6.8, 2 systems 0.72.  The solve runs at about 70 %
+// of the FP64 matrix rate; the factorization is bound by the latency of its pivot
+// steps (0.6 to 0.9 us: the updates and keys of 16 registers 0.25, candidates,
+// barrier and winner 0.2, reciprocal 0.1) and of a panel's loads and products.
 // Error: forward error as an LU's; the residual of an ill-conditioned system can
 // be larger (Gauss-Jordan is not row-wise backward stable), so it serves the
 // systems that are well conditioned by construction.
@@ -43,22 +46,6 @@ namespace {
 typedef double gj_d4 __attribute__((ext_vector_type(4)));
 constexpr int NB = 16;      // panel width
 constexpr int YS = NB + 1;  // LDS row stride
-
-// maximum over the 64 lanes (DPP: inside rows of 16, then across the rows)
-__device__ __forceinline__ int wave_max_int(int v) {
-  int t;
-#define GJ_STEP(ctrl, rmask)                                      \
-  t = __builtin_amdgcn_update_dpp(v, v, ctrl, rmask, 0xf, false); \
-  v = t > v ? t : v;
-  GJ_STEP(0x111, 0xf)  // row_shr:1
-  GJ_STEP(0x112, 0xf)  // row_shr:2
-  GJ_STEP(0x114, 0xf)  // row_shr:4
-  GJ_STEP(0x118, 0xf)  // row_shr:8
-  GJ_STEP(0x142, 0xa)  // row_bcast:15
-  GJ_STEP(0x143, 0xc)  // row_bcast:31
-#undef GJ_STEP
-  return __builtin_amdgcn_readlane(v, 63);
-}
 
 // 1 / v for any finite v: scaled by a power of two, Newton steps on the
 // hardware's reciprocal, no branch (all lanes take it while the pivot search
@@ -184,41 +171,136 @@ __device__ __forceinline__ void apply_panels(Strip<RB, CB>& x, const cd* __restr
 }
 
 // ------------------------------------------------------------ factorization
-// A wavefront's candidate for the pivot of a step.
-struct Candidate {
-  lcd row[NB];
-  lcd recip;
-};
 constexpr int GJ_MAX_WAVES = 8;
+constexpr int ROW_BITS = 9;                                    // rows < GJ_MAX_N
+constexpr int KEY_MASK = 0x7fffffff & ~((1 << ROW_BITS) - 1);  // a key's magnitude bits
+constexpr int CLOSED = (int)0x80000000;
+
+// lane JJ of every 16 lanes to all of them
+template <int JJ>
+__device__ __forceinline__ double bcast16(double v) {
+  return __longlong_as_double(__builtin_amdgcn_mov_dpp(__double_as_longlong(v), 0x150 + JJ, 0xf, 0xf, true));
+}
+
+// every lane's value to the lane four down, around the 16
+__device__ __forceinline__ double rotate4(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x12c, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x12c, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// The panel under elimination, where the matrix cores left it: entry i = 4 t + r
+// of lane l is row 16 t + l / 16 + 4 r of the wavefront, column l % 16.  Vectors,
+// so that a row found at run time is one indexed register move.
+template <int RB>
+struct PanelRegs {
+  typedef double vec __attribute__((ext_vector_type(RB == 3 ? 16 : 4 * RB)));
+  typedef int ivec __attribute__((ext_vector_type(RB == 3 ? 16 : 4 * RB)));
+  vec re, im;
+  // row number, with the sign bit set once the row has been a pivot (or is none)
+  ivec tag;
+};
+
+// A row's key for being the pivot of this lane's column: the high bits of |re| +
+// |im| (to 2^-11), then the row number.
+__device__ __forceinline__ int pivot_key(double re, double im, int tag) {
+  return (__double2hiint(fabs(re) + fabs(im)) & KEY_MASK) | tag;
+}
+
+// the maximum of column JJ's lanes
+template <int JJ>
+__device__ __forceinline__ int column_max(int key) {
+  const int a = max(__builtin_amdgcn_readlane(key, JJ), __builtin_amdgcn_readlane(key, 16 + JJ));
+  const int b = max(__builtin_amdgcn_readlane(key, 32 + JJ), __builtin_amdgcn_readlane(key, 48 + JJ));
+  return max(a, b);
+}
+
+struct FactorLds {
+  lcd* cand;  // 2 x GJ_MAX_WAVES rows of 16 and a spare one
+  int* keys;  // 2 x GJ_MAX_WAVES
+};
+
+// Column k, which lanes JJ of each 16 hold.  best: the wavefront's key for it, then
+// for the next column's; sc: what this lane's column is multiplied with at the
+// end of the panel; pivot: the row this lane's column was eliminated with.
+template <int RB, int JJ>
+__device__ __forceinline__ void eliminate(PanelRegs<RB>& x, int& best, cd& sc, int& pivot, int& first_zero, int k,
+                                          const FactorLds& sm, int nw, int wave, int row0, int li, int lk) {
+  constexpr int buf = (JJ & 1) * GJ_MAX_WAVES;
+  {
+    const int at = (best & ((1 << ROW_BITS) - 1)) - row0;
+    const int i = at >> 2;
+    // (the other rows' lanes write to a spare row, and all lanes the key: no branches)
+    sm.cand[(lk == (at & 3) ? buf + wave : 2 * GJ_MAX_WAVES) * 16 + li] = lcd{x.re[i], x.im[i]};
+    sm.keys[buf + wave] = best;
+  }
+  __syncthreads();
+  int kbest = best;
+  if (nw > 1) {
+    const int4 a = *reinterpret_cast<const int4*>(sm.keys + buf), b = *reinterpret_cast<const int4*>(sm.keys + buf + 4);
+    kbest = __builtin_amdgcn_readfirstlane(max(max(max(a.x, a.y), max(a.z, a.w)), max(max(b.x, b.y), max(b.z, b.w))));
+  }
+  const int prow = kbest & ((1 << ROW_BITS) - 1);
+  const int w = prow / (16 * RB);
+  const lcd pl = sm.cand[(buf + w) * 16 + li];
+  const cd p = mkc(pl.x, pl.y);
+  if ((kbest & KEY_MASK) == 0 && first_zero == 0) first_zero = k + 1;
+  const cd mine = recip_pivot(p);
+  const cd rc = mkc(bcast16<JJ>(mine.x), bcast16<JJ>(mine.y));
+  cd y = p * rc;
+  const bool own = li == JJ;
+  y.x = own ? 0.0 : y.x;  // the column itself stays, until it is scaled with sc
+  y.y = own ? 0.0 : y.y;
+  sc.x = own ? -rc.x : sc.x;
+  sc.y = own ? -rc.y : sc.y;
+  pivot = own ? prow : pivot;
+  // (no branch on whether the row is this wavefront's: the registers would be
+  // copied where its two sides join)
+  const int at = w == wave ? prow - row0 : 0, ip = at >> 2;
+  const bool hit = w == wave && lk == (at & 3);
+  const int tp = x.tag[ip];
+  x.tag[ip] = hit ? CLOSED | prow : tp;
+  int key = CLOSED;
+#pragma unroll
+  for (int i = 0; i < 4 * RB; ++i) {
+    const double mr = bcast16<JJ>(x.re[i]), mi = bcast16<JJ>(x.im[i]);
+    x.re[i] = fma(mi, y.y, fma(-mr, y.x, x.re[i]));
+    x.im[i] = fma(-mi, y.x, fma(-mr, y.y, x.im[i]));
+    const int c = pivot_key(x.re[i], x.im[i], x.tag[i]);
+    key = i == 0 ? c : max(key, c);
+  }
+  const double pr = x.re[ip], pi = x.im[ip];  // the pivot row
+  x.re[ip] = hit ? (own ? -1.0 : y.x) : pr;
+  x.im[ip] = hit ? y.y : pi;
+  best = column_max<JJ + 1>(key);
+}
 
 // Columns c0 .. c1 - 1 (c0 a multiple of 16), to which the panels before c0 have
-// been applied.  Workgroups of ceil(n / (16 RB)) wavefronts; in the elimination
-// lane l of wavefront w owns row 16 RB w + l (l < 16 RB).
+// been applied.  Workgroups of ceil(n / (16 RB)) wavefronts.
 template <int RB>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3 : 2))) void gj_factor_kernel(int n, int c0, int c1, cd* A, int lda, long long sA, int* perm, int* info) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3 : 2))) void gj_factor_kernel(
+    int n, int c0, int c1, cd* A, int lda, long long sA, int* perm, int* info) {
   extern __shared__ lcd sm[];
   const int nw = blockDim.x >> 6;
-  lcd* stage = sm;                                                         // nw x 16 x YS, wavefront-private
-  lcd* Y = stage + nw * 16 * YS;                                           // 2 x 17 x YS
-  Candidate* cand = reinterpret_cast<Candidate*>(Y + 2 * (NB + 1) * YS);   // 2 x 8
-  int4* keys = reinterpret_cast<int4*>(cand + 2 * GJ_MAX_WAVES);           // 2 x 8 (key, row) pairs
-  int* ord = reinterpret_cast<int*>(keys + GJ_MAX_WAVES);                  // 16 RB nw
+  lcd* Y = sm;  // 2 x 17 x YS
+  FactorLds fl;
+  fl.cand = Y + 2 * (NB + 1) * YS;
+  fl.keys = reinterpret_cast<int*>(fl.cand + (2 * GJ_MAX_WAVES + 1) * 16);
+  int* ord = fl.keys + 2 * GJ_MAX_WAVES;  // 16 RB nw
   const long long item = blockIdx.x;
   cd* a = A + item * sA;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lk = lane >> 4;
   const int row0 = wave * 16 * RB;
-  const int row = lane < 16 * RB ? row0 + lane : n;  // the row this lane eliminates
   int first_zero = 0;
   for (int e = tid; e < 16 * RB * nw; e += blockDim.x) ord[e] = 1 << 30;
-  if (tid < GJ_MAX_WAVES) keys[tid] = make_int4(-2, 0, -2, 0);
+  if (tid < 2 * GJ_MAX_WAVES) fl.keys[tid] = CLOSED;
   __syncthreads();
   for (int k = tid; k < c0; k += blockDim.x) ord[perm[item * n + k]] = k;
   __syncthreads();
-  bool open = row < n && ord[min(row, n - 1)] == 1 << 30;
   for (int k0 = c0; k0 < c1; k0 += NB) {
     const int nb = min(NB, n - k0);
-    cd x[NB];
+    PanelRegs<RB> x;
     {
       // (rows past n and columns past the last panel's: the edge's values, which
       // reach nothing that is stored)
@@ -233,108 +315,52 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 3 ? 3
           st.re[t][0][r] = v.x;
           st.im[t][0][r] = v.y;
           st.slot[t][r] = ord[gr];
+          x.tag[4 * t + r] = gr | (gr < n && st.slot[t][r] == 1 << 30 ? 0 : CLOSED);
         }
       apply_panels(st, a, lda, n, c0 / NB, k0 / NB, NB, Y, row0, li, lk);
-      // accumulators -> one row per lane, 16 rows at a time through the
-      // wavefront's own LDS
-      lcd* sp = stage + wave * 16 * YS;
 #pragma unroll
-      for (int c = 0; c < NB; ++c) x[c] = mkc(0.0, 0.0);
+      for (int t = 0; t < RB; ++t)
 #pragma unroll
-      for (int t = 0; t < RB; ++t) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sp[(lk + 4 * r) * YS + li] = lcd{st.re[t][0][r], st.im[t][0][r]};
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (lk == t) {
-#pragma unroll
-          for (int c = 0; c < NB; ++c) x[c] = mkc(sp[li * YS + c].x, sp[li * YS + c].y);
+        for (int r = 0; r < 4; ++r) {
+          x.re[4 * t + r] = st.re[t][0][r];
+          x.im[4 * t + r] = st.im[t][0][r];
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-      }
     }
-    // Eliminate the panel's columns.  The columns rotate through x: the current
-    // one is x[0], the others move down by one as they are updated and the
-    // finished column enters at the end, so one loop body serves every step and
-    // sixteen steps restore the order.
-    // key: the high word of |re| + |im| orders the candidates to 2^-20; rows
-    // already used have -1
-    int key = open ? __double2hiint(cabs1(x[0])) & 0x7fffffff : -1;
-    cd rc = recip_pivot(x[0]);
-    int best = wave_max_int(key);
+    int key = 0;
+#pragma unroll
+    for (int i = 0; i < 4 * RB; ++i) {
+      const int c = pivot_key(x.re[i], x.im[i], x.tag[i]);
+      key = i == 0 ? c : max(key, c);
+    }
+    cd sc = mkc(0.0, 0.0);
+    int best = column_max<0>(key), col = li, pivot = 0;
+    // Four columns per pass through the code, then the columns move four lanes
+    // down: which lane is read is part of the instruction, and sixteen copies of
+    // the step (50 KB) would be fetched more slowly than they run.
 #pragma unroll 1
-    for (int jj = 0; jj < nb; ++jj) {
-      const int buf = (jj & 1) * GJ_MAX_WAVES;
-      const int src = __ffsll((unsigned long long)__ballot(key == best)) - 1;
-      if (lane == src) {
-        Candidate& c = cand[buf + wave];
-        reinterpret_cast<int2*>(keys)[buf + wave] = make_int2(best, row);
+    for (int j = 0; j < nb; j += 4) {
+      eliminate<RB, 0>(x, best, sc, pivot, first_zero, k0 + j, fl, nw, wave, row0, li, lk);
+      if (j + 1 < nb) eliminate<RB, 1>(x, best, sc, pivot, first_zero, k0 + j + 1, fl, nw, wave, row0, li, lk);
+      if (j + 2 < nb) eliminate<RB, 2>(x, best, sc, pivot, first_zero, k0 + j + 2, fl, nw, wave, row0, li, lk);
+      if (j + 3 < nb) eliminate<RB, 3>(x, best, sc, pivot, first_zero, k0 + j + 3, fl, nw, wave, row0, li, lk);
 #pragma unroll
-        for (int q = 0; q < NB; ++q) c.row[q] = lcd{x[q].x, x[q].y};
-        c.recip = lcd{rc.x, rc.y};
+      for (int i = 0; i < 4 * RB; ++i) {
+        x.re[i] = rotate4(x.re[i]);
+        x.im[i] = rotate4(x.im[i]);
       }
-      __syncthreads();
-      int w = 0, kbest = best, prow = row0 + src;
-      if (nw > 1) {
-        int4 kq[GJ_MAX_WAVES / 2];
-#pragma unroll
-        for (int q = 0; q < GJ_MAX_WAVES / 2; ++q) kq[q] = keys[buf / 2 + q];
-        kbest = kq[0].x;
-        prow = kq[0].y;
-#pragma unroll
-        for (int q = 1; q < GJ_MAX_WAVES; ++q) {
-          const int k = q & 1 ? kq[q / 2].z : kq[q / 2].x, r = q & 1 ? kq[q / 2].w : kq[q / 2].y;
-          const bool more = k > kbest;
-          w = more ? q : w;
-          prow = more ? r : prow;
-          kbest = more ? k : kbest;
-        }
-        w = __builtin_amdgcn_readfirstlane(w);
-      }
-      const Candidate& c = cand[buf + w];
-      const lcd rp = c.recip;
-      lcd pa[8], pb[7];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) pa[q] = c.row[q + 1];
-      __builtin_amdgcn_sched_barrier(0);  // half of the row is on its way before the first use
-      if (kbest == 0 && first_zero == 0) first_zero = k0 + jj + 1;
-      cd m = x[0] * mkc(rp.x, rp.y);
-      if (row == prow) {
-        open = false;
-        ord[row] = k0 + jj;
-        m = mkc(-rp.x, -rp.y);
-#pragma unroll
-        for (int q = 0; q < NB; ++q) x[q] = mkc(0.0, 0.0);
-      }
-      // the next column first: its pivot search and reciprocals run beside the
-      // other columns' updates
-      x[0] = fmsc(x[1], m, mkc(pa[0].x, pa[0].y));
-      key = open ? __double2hiint(cabs1(x[0])) & 0x7fffffff : -1;
-#pragma unroll
-      for (int q = 0; q < 7; ++q) pb[q] = c.row[q + 9];
-      rc = recip_pivot(x[0]);
-      best = wave_max_int(key);
-#pragma unroll
-      for (int q = 1; q < 8; ++q) x[q] = fmsc(x[q + 1], m, mkc(pa[q].x, pa[q].y));
-#pragma unroll
-      for (int q = 8; q < NB - 1; ++q) x[q] = fmsc(x[q + 1], m, mkc(pb[q - 8].x, pb[q - 8].y));
-      x[NB - 1] = -m;
+      sc = mkc(rotate4(sc.x), rotate4(sc.y));
+      pivot = __builtin_amdgcn_mov_dpp(pivot, 0x12c, 0xf, 0xf, true);
+      col = (col + 4) & 15;
     }
-    for (int jj = nb; jj < NB; ++jj) {  // the last panel: rotate on
-      const cd t = x[0];
+    if (wave + lk == 0 && col < nb) ord[pivot] = k0 + col;
 #pragma unroll
-      for (int q = 1; q < NB; ++q) x[q - 1] = x[q];
-      x[NB - 1] = t;
-    }
-    if (row < n) {
-#pragma unroll
-      for (int c = 0; c < NB; ++c)
-        if (c < nb) a[(unsigned)(row * lda + k0 + c)] = x[c];
+    for (int i = 0; i < 4 * RB; ++i) {
+      const int gr = row0 + 4 * i + lk;
+      if (gr < n && col < nb) a[(unsigned)(gr * lda + k0 + col)] = mkc(x.re[i], x.im[i]) * sc;
     }
     __syncthreads();  // G and ord of this panel are read by the other wavefronts
   }
-  if (row < n) {
+  for (int row = tid; row < n; row += blockDim.x) {
     const int k = ord[row];
     if (k >= c0 && k < c1) perm[item * n + k] = row;
   }
@@ -438,8 +464,8 @@ int strips_sized(hipStream_t s, int n, int m, int j0, int j1, Mat A, Mat B, int 
 template <int RB>
 int launch_factor(hipStream_t s, int n, int c0, int c1, Mat A, int batch, int* perm, int* info) {
   const int nw = (n + 16 * RB - 1) / (16 * RB);
-  const size_t lds = (size_t)(nw * 16 + 2 * (NB + 1)) * YS * sizeof(lcd) + 2 * GJ_MAX_WAVES * (sizeof(Candidate) + sizeof(int2)) +
-                     (size_t)nw * 16 * RB * sizeof(int);
+  const size_t lds = ((size_t)2 * (NB + 1) * YS + (2 * GJ_MAX_WAVES + 1) * 16) * sizeof(lcd) +
+                     ((size_t)2 * GJ_MAX_WAVES + nw * 16 * RB) * sizeof(int);
   KHX_TRY(ensure_dynamic_lds((const void*)gj_factor_kernel<RB>, lds));
   gj_factor_kernel<RB><<<dim3((unsigned)batch), dim3(64 * nw), lds, s>>>(n, c0, c1, A.p, A.ld, A.stride, perm, info);
   KHX_LAUNCH_CHECK();
@@ -462,25 +488,29 @@ int zgj_solve(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* perm, i
   ProfScope ps("zgesv_kernel", s);
   // Columns factored by one launch before the others are brought up to date.  One
   // workgroup per system factors, so few systems leave most of the chip to the
-  // updates' strips, and panels of a launch that reads back little cost little:
-  // 64 columns below 256 systems (n = 338, 16 systems: 1.01 ms against 1.14 with
-  // 128 and 1.82 in one launch; n = 162, 64: 0.37 / 0.38 / 0.40).  Beyond, the CUs
-  // are full either way: 128 columns where G outgrows what a CU's cache keeps
-  // (n = 338, 512 systems: 7.4 / 7.1 / 7.5 ms), all at once up to n = 192 (n =
-  // 162, 1 024: 2.06 / 1.99 / 1.90).
-  const int wb = batch < 256 ? 64 : n > 192 ? 128 : n;
-  // Rows per wavefront of the factorization: 64 while one or two wavefronts hold
-  // the matrix (fewer barriers per pivot; n = 98, 1 000 systems: 0.56 ms against
-  // 0.72 with 48), 48 where 64 would leave three wavefronts on four SIMDs (n =
-  // 162, 2 048: 3.7 against 4.0 ms), 64 again where four or more are needed
-  // (n = 338, 48: 1.48 against 1.53 ms).
-  const int rbf = n > 128 && n <= 192 ? 3 : 4;
+  // updates' strips: 32 columns up to 32 systems (from n = 129; n = 338, 2 systems:
+  // 0.72 ms against 0.77 with 64 and 1.6 in one launch), 64 below 256 (n = 338, 64:
+  // 1.45 / 1.49 / 1.52 ms with 64 / 32 / 128; n = 162, 64: 0.30 / 0.31 / 0.32).
+  // Beyond, the CUs are full either way: 128 columns where G outgrows what a CU's
+  // cache keeps (n = 338, 512 systems: 7.1 / 6.8 / 7.2 ms with 64 / 128 / all), all
+  // at once up to n = 192 (n = 162, 1 024: 1.94 / 1.90 / 1.87).
+  const int wb = batch <= 32 && n > 128 ? 32 : batch < 256 ? 64 : n > 192 ? 128 : n;
+  // Rows per wavefront of the factorization, 16 rb.  A step's updates go with rb,
+  // the rest of it with the wavefronts: four wavefronts on the four SIMDs while a
+  // CU has one or two systems (n = 50, 128 systems: 0.061 ms against 0.076 in one
+  // wavefront; n = 98, 128: 0.154 / 0.17), as few as hold the matrix beyond (n =
+  // 50, 2 048: 0.25 / 0.20; n = 98, 1 000: 0.55 / 0.53).  n = 162 in four
+  // wavefronts of 48 rows when the CUs are full (512 systems: 0.94 against 0.98).
+  const bool full = batch > 512;
+  const int rbf = n <= 64 ? (full ? 4 : 1) : n <= 128 ? (full ? 4 : 2) : n <= 192 && batch >= 256 ? 3 : 4;
   for (int c0 = 0; c0 < n; c0 += wb) {
     const int c1 = c0 + wb < n ? c0 + wb : n;
-    if (rbf == 3)
-      KHX_TRY(launch_factor<3>(s, n, c0, c1, A, batch, perm, info));
-    else
-      KHX_TRY(launch_factor<4>(s, n, c0, c1, A, batch, perm, info));
+    switch (rbf) {
+      case 1: KHX_TRY(launch_factor<1>(s, n, c0, c1, A, batch, perm, info)); break;
+      case 2: KHX_TRY(launch_factor<2>(s, n, c0, c1, A, batch, perm, info)); break;
+      case 3: KHX_TRY(launch_factor<3>(s, n, c0, c1, A, batch, perm, info)); break;
+      default: KHX_TRY(launch_factor<4>(s, n, c0, c1, A, batch, perm, info));
+    }
     if (c1 < n)
       KHX_TRY(strips_sized<false>(s, n, n - c1, c0 / NB, c1 / NB, A, Mat{A.p + c1, A.ld, A.stride}, batch, perm));
   }

@@ -68,16 +68,20 @@ def test_singular_and_nan_items(gpu, n):
         assert np.linalg.norm(X[b] - ref) <= 64e-16 * n * np.linalg.cond(A[b]) * np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("n,m,batch", [(192, 9, 256), (193, 17, 255), (193, 17, 256), (256, 3, 256), (257, 40, 257)])
-def test_columns_in_several_launches(gpu, n, m, batch):
-    """Around the batch and the order from which 64, 128 or all columns are
-    factored by one launch; a zero column in a later launch is reported."""
+@pytest.mark.parametrize("n,m,batch", [
+    (15, 3, 513), (64, 5, 513), (100, 4, 513), (129, 20, 33), (192, 9, 256), (193, 17, 255), (193, 17, 256),
+    (256, 3, 256), (257, 40, 257)])
+def test_columns_and_rows_by_batch(gpu, n, m, batch):
+    """Around the batches and orders where the columns of a launch (32, 64, 128,
+    all) and the rows of a wavefront change; a zero column, in a later launch
+    where there are several, is reported."""
     rng = np.random.default_rng(n + batch)
     A = rng.normal(size=(batch, n, n)) + 1j * rng.normal(size=(batch, n, n))
     B = rng.normal(size=(batch, n, m)) + 1j * rng.normal(size=(batch, n, m))
-    A[1, :, 150] = 0.0
+    zero = 3 * n // 4
+    A[1, :, zero] = 0.0
     X, info = _solve(A, B, gpu)
-    assert info[1] == 151 and (np.delete(info, 1) == 0).all()
+    assert info[1] == zero + 1 and (np.delete(info, 1) == 0).all()
     for b in (0, batch // 2, batch - 1):
         ref = np.linalg.solve(A[b], B[b])
         err = np.linalg.norm(X[b] - ref) / np.linalg.norm(ref)
