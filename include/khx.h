@@ -225,8 +225,8 @@ int khx_halfspace(int side, const double* kx, const double* ky, int N, int batch
 size_t khx_redheffer_ws_bytes(int n, int batch);
 int khx_redheffer(const double* SA, int a_bcast, const double* SB, int b_bcast, int n, int batch, double* S,
                   int* info, void* ws, void* stream);
-/* The same with both solves in one batch of khx_zgesv_ws's kind (two launches,
- * Gauss-Jordan); where fields are read from the chain use khx_redheffer.   */
+/* The same with one solve of khx_zgesv_ws's kind (info: first zero pivot of D);
+ * where fields are read from the chain use khx_redheffer.                  */
 int khx_redheffer_gj(const double* SA, int a_bcast, const double* SB, int b_bcast, int n, int batch, double* S,
                      int* info, void* ws, void* stream);
 

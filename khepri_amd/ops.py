@@ -567,8 +567,8 @@ def analytic_layer(kind, kx, ky, eps, k0d=None, modes=False):
 
 
 def redheffer(SA, SB, out=None, ws=None, gj=False):
-    """SA * SB, with its status words; gj: the two solves through
-    khx_zgesv_ws's Gauss-Jordan in one batch -- for chains that only R, T or S
+    """SA * SB, with its status words; gj: one solve, through
+    khx_zgesv_ws's Gauss-Jordan -- for chains that only R, T or S
     are read from (a chain that fields or gradients are read from keeps the LU)."""
     lib = _lib.load()
     ab = SA.dim() == 4

@@ -86,3 +86,28 @@ def test_columns_and_rows_by_batch(gpu, n, m, batch):
         ref = np.linalg.solve(A[b], B[b])
         err = np.linalg.norm(X[b] - ref) / np.linalg.norm(ref)
         assert err <= 64e-16 * n * np.linalg.cond(A[b]), (b, err)
+
+
+@pytest.mark.parametrize("n,batch,wide", [(2, 3, "neither"), (18, 40, "a"), (50, 2, "b"), (530, 2, "neither")])
+def test_star_product_with_one_solve(gpu, n, batch, wide):
+    """redheffer(gj=True) against the formula with two solves, per item and with
+    either operand shared by the batch.  Blocks of norm ~1/2: cond(D) < 2, so the
+    products' rounding is all there is (64 n eps)."""
+    import torch
+    from khepri_amd import ops
+    rng = np.random.default_rng(n)
+
+    def draw(count):
+        S = rng.normal(size=(count, 2, 2, n, n)) + 1j * rng.normal(size=(count, 2, 2, n, n))
+        return S / (4 * np.sqrt(2 * n))
+    A, B = draw(1 if wide == "a" else batch), draw(1 if wide == "b" else batch)
+    put = lambda S: torch.as_tensor(S[0] if wide != "neither" and len(S) == 1 else S, device=gpu)   # noqa: E731
+    S, info = ops.redheffer(put(A), put(B), gj=True)
+    assert (info.cpu().numpy() == 0).all()
+    S = S.cpu().numpy()
+    for b in (0, batch - 1):
+        a, c = A[b % len(A)], B[b % len(B)]
+        D, F = np.eye(n) - c[0, 0] @ a[1, 1], np.eye(n) - a[1, 1] @ c[0, 0]
+        ref = np.array([[a[0, 0] + a[0, 1] @ np.linalg.solve(D, c[0, 0]) @ a[1, 0], a[0, 1] @ np.linalg.solve(D, c[0, 1])],
+                        [c[1, 0] @ np.linalg.solve(F, a[1, 0]), c[1, 1] + c[1, 0] @ np.linalg.solve(F, a[1, 1]) @ c[0, 1]]])
+        assert np.linalg.norm(S[b] - ref) <= 64e-16 * n * np.linalg.norm(ref)
