@@ -124,22 +124,30 @@ static int launch_zgemm(hipStream_t s, int M, int N, int K, cd alpha, Mat A, Mat
 // A complex product is four real ones: Re += Ar Br - Ai Bi, Im += Ar Bi + Ai Br.
 // A workgroup (4 wavefronts in a 2 x 2 grid) owns a (32 WM) x (32 WN) tile of
 // C; each wavefront owns WM x WN blocks of 16 x 16.  K advances 16 at a time
-// through LDS (k-major, one complex of padding per row against bank
-// conflicts); the next K slice is fetched into registers while the current
-// one is multiplied.  Consecutive tiles of one batch item are kept on one XCD
-// (workgroups are dealt round-robin to the 8 XCDs) so they share its L2.
+// through one of two LDS buffers (k-major, one complex of padding per row against
+// bank conflicts; one barrier per slice); the next K slice is fetched into
+// registers while the current one is multiplied.  Consecutive tiles of one batch
+// item are kept on one XCD (workgroups are dealt round-robin to the 8 XCDs) so they
+// share its L2.
+// Bound by the matrix cores, which share their issue with everything else: the
+// accumulators have to stay in VGPRs over the loop (two wavefronts per SIMD or more
+// in the launch bounds: else they are kept in AGPRs and copied at every slice, 64
+// moves and the wait for the last product), and a tile's blocks and k past the edge
+// are left out.  512 products of n = 162 38 -> 45 TF, 24 of 338 41 -> 55, 8 of 1 250
+// 57 -> 63 of the 73 that a large product reaches; the sums are in the same order.
 typedef double khx_d4 __attribute__((ext_vector_type(4)));
 
 template <int WM, int WN, int OA, int OB>
-__global__ __launch_bounds__(256) void zgemm_mfma_kernel(int M, int N, int K, cd alpha,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WM * WN > 2 ? 2 : 3))) void
+zgemm_mfma_kernel(int M, int N, int K, cd alpha,
                                                          const cd* __restrict__ A, int lda, long long sA,
                                                          const cd* __restrict__ B, int ldb, long long sB,
                                                          cd beta, cd* __restrict__ C, int ldc, long long sC,
                                                          int tilesN, int tilesPerItem, int xcd_remap) {
   constexpr int BM = 32 * WM, BN = 32 * WN, BK = 16;
   constexpr int LA = (BM * BK) / 256, LBn = (BK * BN) / 256;  // complex loads per thread
-  __shared__ cd As[BK][BM + 1];
-  __shared__ cd Bs[BK][BN + 1];
+  __shared__ cd As[2][BK][BM + 1];
+  __shared__ cd Bs[2][BK][BN + 1];
 
   unsigned bid = blockIdx.x;
   if (xcd_remap) {  // gridDim.x % 8 == 0: logical tile order = XCD-major
@@ -150,12 +158,13 @@ __global__ __launch_bounds__(256) void zgemm_mfma_kernel(int M, int N, int K, cd
   const int tile = bid % tilesPerItem;
   const int row0 = (tile / tilesN) * BM;
   const int col0 = (tile % tilesN) * BN;
-  const cd* a = A + item * sA;
-  const cd* b = B + item * sB;
   cd* c = C + item * sC;
 
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63;
+  // (which wavefront has which quarter of the tile goes round with the tiles, so
+  // that a partial tile's idle quarters do not all fall to the same SIMD)
+  const int wave = __builtin_amdgcn_readfirstlane(((tid >> 6) + bid) & 3);
   const int wr = (wave >> 1) * (16 * WM), wc = (wave & 1) * (16 * WN);
   const int li = lane & 15, lk = lane >> 4;
 
@@ -168,66 +177,125 @@ __global__ __launch_bounds__(256) void zgemm_mfma_kernel(int M, int N, int K, cd
       accI[t][u] = khx_d4{0.0, 0.0, 0.0, 0.0};
     }
 
+  // Rows of A and columns of B past the edge are read from the edge: what they
+  // give is not stored.
+  const cd *pa[LA], *pb[LBn];
+#pragma unroll
+  for (int q = 0; q < LA; ++q) {
+    const int e = tid + 256 * q;
+    const int r = OA ? e % BM : e / BK, kk = OA ? e / BM : e % BK;
+    const int gr = min(row0 + r, M - 1);
+    pa[q] = A + item * sA + (OA ? (long long)kk * lda + gr : (long long)gr * lda + kk);
+  }
+#pragma unroll
+  for (int q = 0; q < LBn; ++q) {
+    const int e = tid + 256 * q;
+    const int kk = OB ? e % BK : e / BN, cc = OB ? e / BK : e % BN;
+    const int gc = min(col0 + cc, N - 1);
+    pb[q] = B + item * sB + (OB ? (long long)gc * ldb + kk : (long long)kk * ldb + gc);
+  }
+  const long long stepA = OA ? (long long)BK * lda : BK, stepB = OB ? BK : (long long)BK * ldb;
   cd ra[LA], rb[LBn];
-  auto fetch = [&](int k0) {
+  auto fetch = [&]() {  // a whole slice
+#pragma unroll
+    for (int q = 0; q < LA; ++q) {
+      ra[q] = *pa[q];
+      pa[q] += stepA;
+    }
+#pragma unroll
+    for (int q = 0; q < LBn; ++q) {
+      rb[q] = *pb[q];
+      pb[q] += stepB;
+    }
+  };
+  auto fetch_part = [&](int left) {  // the last, of `left` k: the others are 0
+#pragma unroll
+    for (int q = 0; q < LA; ++q) {
+      const int e = tid + 256 * q, kk = OA ? e / BM : e % BK;
+      ra[q] = kk < left ? *pa[q] : mkc(0.0, 0.0);
+    }
+#pragma unroll
+    for (int q = 0; q < LBn; ++q) {
+      const int e = tid + 256 * q, kk = OB ? e % BK : e / BN;
+      rb[q] = kk < left ? *pb[q] : mkc(0.0, 0.0);
+    }
+  };
+  int buf = 1;
+  // the fetched slice to the other LDS buffer (two of them: one barrier per slice)
+  auto stage = [&]() {
+    buf ^= 1;
 #pragma unroll
     for (int q = 0; q < LA; ++q) {
       const int e = tid + 256 * q;
       const int r = OA ? e % BM : e / BK, kk = OA ? e / BM : e % BK;
-      const int gr = row0 + r, gk = k0 + kk;
-      const long long off = OA ? (long long)gk * lda + gr : (long long)gr * lda + gk;
-      cd v = (gr < M && gk < K) ? a[off] : mkc(0.0, 0.0);
-      if (OA == 2) v.y = -v.y;
-      ra[q] = v;
+      As[buf][kk][r] = OA == 2 ? mkc(ra[q].x, -ra[q].y) : ra[q];
     }
 #pragma unroll
     for (int q = 0; q < LBn; ++q) {
       const int e = tid + 256 * q;
       const int kk = OB ? e % BK : e / BN, cc = OB ? e / BK : e % BN;
-      const int gk = k0 + kk, gc = col0 + cc;
-      const long long off = OB ? (long long)gc * ldb + gk : (long long)gk * ldb + gc;
-      cd v = (gk < K && gc < N) ? b[off] : mkc(0.0, 0.0);
-      if (OB == 2) v.y = -v.y;
-      rb[q] = v;
+      Bs[buf][kk][cc] = OB == 2 ? mkc(rb[q].x, -rb[q].y) : rb[q];
+    }
+    __syncthreads();
+  };
+  auto multiply = [&](int kq) {
+    cd av[WM], bv[WN];
+#pragma unroll
+    for (int t = 0; t < WM; ++t) av[t] = As[buf][kq * 4 + lk][wr + t * 16 + li];
+#pragma unroll
+    for (int u = 0; u < WN; ++u) bv[u] = Bs[buf][kq * 4 + lk][wc + u * 16 + li];
+#pragma unroll
+    for (int t = 0; t < WM; ++t)
+#pragma unroll
+      for (int u = 0; u < WN; ++u) {
+        accR[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t].x, bv[u].x, accR[t][u], 0, 0, 0);
+        accI[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t].x, bv[u].y, accI[t][u], 0, 0, 0);
+      }
+#pragma unroll
+    for (int t = 0; t < WM; ++t) {
+      const double nai = -av[t].y;
+#pragma unroll
+      for (int u = 0; u < WN; ++u) {
+        accR[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, bv[u].y, accR[t][u], 0, 0, 0);
+        accI[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t].y, bv[u].x, accI[t][u], 0, 0, 0);
+      }
     }
   };
 
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += BK) {
-#pragma unroll
-    for (int q = 0; q < LA; ++q) {
-      const int e = tid + 256 * q;
-      const int r = OA ? e % BM : e / BK, kk = OA ? e / BM : e % BK;
-      As[kk][r] = ra[q];
+  const int whole = K / BK, part = K % BK;
+  if (whole > 0)
+    fetch();
+  else
+    fetch_part(part);
+  // (a wavefront without any of C only helps to stage; its own loop, so that no
+  // accumulators are copied where the two would join)
+  if (row0 + wr >= M || col0 + wc >= N) {
+    for (int s = 0; s < whole; ++s) {
+      stage();
+      if (s + 1 < whole)
+        fetch();
+      else if (part)
+        fetch_part(part);
     }
+    if (part) stage();
+    return;
+  }
+  for (int s = 0; s + 1 < whole; ++s) {
+    stage();
+    fetch();
 #pragma unroll
-    for (int q = 0; q < LBn; ++q) {
-      const int e = tid + 256 * q;
-      const int kk = OB ? e % BK : e / BN, cc = OB ? e / BK : e % BN;
-      Bs[kk][cc] = rb[q];
-    }
-    __syncthreads();
-    if (k0 + BK < K) fetch(k0 + BK);
+    for (int kq = 0; kq < BK / 4; ++kq) multiply(kq);
+  }
+  if (whole > 0) {
+    stage();
+    if (part) fetch_part(part);
 #pragma unroll
-    for (int kq = 0; kq < BK / 4; ++kq) {
-      cd av[WM], bv[WN];
-#pragma unroll
-      for (int t = 0; t < WM; ++t) av[t] = As[kq * 4 + lk][wr + t * 16 + li];
-#pragma unroll
-      for (int u = 0; u < WN; ++u) bv[u] = Bs[kq * 4 + lk][wc + u * 16 + li];
-#pragma unroll
-      for (int t = 0; t < WM; ++t) {
-        const double nai = -av[t].y;
-#pragma unroll
-        for (int u = 0; u < WN; ++u) {
-          accR[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t].x, bv[u].x, accR[t][u], 0, 0, 0);
-          accR[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, bv[u].y, accR[t][u], 0, 0, 0);
-          accI[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t].x, bv[u].y, accI[t][u], 0, 0, 0);
-          accI[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t].y, bv[u].x, accI[t][u], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
+    for (int kq = 0; kq < BK / 4; ++kq) multiply(kq);
+  }
+  if (part) {
+    stage();
+#pragma unroll 1
+    for (int kq = 0; 4 * kq < part; ++kq) multiply(kq);
   }
 
   const bool use_beta = (beta.x != 0.0 || beta.y != 0.0);
@@ -407,8 +475,12 @@ int zgemm_f32(hipStream_t s, int M, int N, int K, cd alpha, Mat A, Mat B, cd bet
 // ---- tile selection.  Eight kernels (all 256 threads): FMA tiles
 //   0: 64 x 64 (4 x 4 per thread), 1: 32 x 32 (2 x 2), 2: 64 x 32 (4 x 2), 3: 32 x 64 (2 x 4);
 // MFMA tiles 4: 64 x 64, 5: 32 x 32, 6: 64 x 32, 7: 32 x 64.
-// The default is MFMA 32 x 32 when a side is at most 96 and MFMA 32 x 64 otherwise
-// (the fastest of the eight on the batched layer shapes); a per-shape choice installed by the
+// The default is MFMA 32 x 32: it leaves the fewest blocks of a partial tile and the
+// most workgroups (n = 338, 24 products: 51 -> 55 TF against 32 x 64, 2 products 21 ->
+// 32 TF; n = 162 times 324 columns, 512: 46 -> 50), and loses at most 3 % where the
+// larger tiles divide the product (n = 242, 512).  Many tiles of operands that no
+// longer fit an L2 want the traffic of MFMA 64 x 64 (1 250 x 2 500 x 1 250, 8 products:
+// 65 against 55 TF; 2 products: 58 against 63).  A per-shape choice installed by the
 // autotuner (khepri_amd/autotune.py, through khx_gemm_tune_set) takes precedence, and
 // khx_gemm_force overrides both while candidates are timed.  With recording on, every
 // distinct (M, N, K, opA, opB, batch class) passing through is kept for the autotuner.
@@ -437,7 +509,8 @@ int gemm_tile_choice(int M, int N, int K, int oa, int ob, int batch) {
   }
   const auto it = g_tune.find(key);
   if (it != g_tune.end()) return it->second;
-  return (M <= 96 || N <= 96) ? 5 : 7;
+  const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
+  return M >= 1024 && N >= 1024 && tiles64 >= 2048 ? 4 : 5;
 }
 
 template <int OA, int OB>
