@@ -488,62 +488,130 @@ __global__ __launch_bounds__(LB_THREADS) void zlu_panel_kernel(int n, int m, int
   panel_apply<NB>(n, m, j0, nb, a, lda, bm, ldb, pan, pld, perm, info, item, first_zero, keepL, cend);
 }
 
+// maximum over the 64 lanes (DPP: inside rows of 16, then across the rows)
+__device__ __forceinline__ int wave_max_int(int v) {
+  int t;
+#define LB_STEP(ctrl, rmask)                                      \
+  t = __builtin_amdgcn_update_dpp(v, v, ctrl, rmask, 0xf, false); \
+  v = t > v ? t : v;
+  LB_STEP(0x111, 0xf)  // row_shr:1
+  LB_STEP(0x112, 0xf)  // row_shr:2
+  LB_STEP(0x114, 0xf)  // row_shr:4
+  LB_STEP(0x118, 0xf)  // row_shr:8
+  LB_STEP(0x142, 0xa)  // row_bcast:15
+  LB_STEP(0x143, 0xc)  // row_bcast:31
+#undef LB_STEP
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// What the wavefronts of a register panel exchange at a pivot step: each one's
+// candidate (|Re| + |Im|, its place, 1 / pivot, its row); two sets in turn.
+template <int NB, int TH>
+struct PanelLds {
+  double best[2][TH / 64];
+  int place[2][TH / 64];
+  cd recip[2][TH / 64];
+  cd row[2][TH / 64][NB];
+  int src[NB];  // the row that ends at place i of the first NB (rows of the panel's start)
+  int dst[NB];  // where row i of the first NB ends
+};
+
 // Pivot step JJ of the register panel (a template parameter, so that every
-// index into the row registers is a constant).
+// index into the row registers is a constant).  pos: the rows' places after the
+// interchanges so far (-1: no row); the rows themselves stay in their threads.
 template <int NB, int RPT, int JJ, int TH>
-__device__ __forceinline__ void panel_step(cd (&v)[RPT][NB], int nb, int pr, int j0, int n, long long item, int* ipiv,
-                                           int* perm, cd* prow, cd* jrow, double* rv, int* ri, cd* rc,
-                                           int& first_zero) {
+__device__ __forceinline__ void panel_step(cd (&v)[RPT][NB], int (&pos)[RPT], int nb, int pr, int j0, int n,
+                                           long long item, int* ipiv, PanelLds<NB, TH>& sm, int& first_zero) {
   if (JJ >= nb) return;  // uniform: the last panel may be narrower
-  const int tid = threadIdx.x;
+  constexpr int buf = JJ & 1, W = TH / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   double best = -1.0;
   int bi = pr;
-  cd bv = mkc(0.0, 0.0);
+  cd bv = mkc(1.0, 0.0);
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
-    const int r = tid + k * TH;
-    if (r >= JJ && r < pr) {
-      const double av = cabs1(v[k][JJ]);
-      if (av > best) {
-        best = av;
-        bi = r;
-        bv = v[k][JJ];
+    const double av = cabs1(v[k][JJ]);
+    if (pos[k] >= JJ && (av > best || (av == best && pos[k] < bi))) {
+      best = av;
+      bi = pos[k];
+      bv = v[k][JJ];
+    }
+  }
+  // the largest of the wavefront, the first place on ties: the high words decide
+  // unless two lanes share the largest
+  const int hi = __double2hiint(best);
+  const int top = wave_max_int(hi);
+  unsigned long long ask = __ballot(hi == top);
+  if (top >= 0 && (ask & (ask - 1))) {
+    double wb = best;
+    int wi = bi;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const double ov = __shfl_xor(wb, o, 64);
+      const int oi = __shfl_xor(wi, o, 64);
+      if (ov > wb || (ov == wb && oi < wi)) {
+        wb = ov;
+        wi = oi;
       }
     }
+    ask = __ballot(bi == wi && best >= 0.0);
   }
-  argmax_abs1<TH>(best, bi, bv, rv, ri, rc);
-  const int p = bi < pr ? bi : JJ;  // NaN column: keep the diagonal
-  // rows p (the new pivot row) and JJ trade places through LDS
+  if (lane == __ffsll(ask) - 1) {
+    sm.best[buf][wid] = best;
+    sm.place[buf][wid] = bi;
 #pragma unroll
-  for (int k = 0; k < RPT; ++k) {
-    const int r = tid + k * TH;
-    if (r == p) {
+    for (int k = 0; k < RPT; ++k)
+      if (RPT == 1 || pos[k] == bi) {
 #pragma unroll
-      for (int c = 0; c < NB; ++c) prow[c] = v[k][c];
-    } else if (r == JJ) {
-#pragma unroll
-      for (int c = 0; c < NB; ++c) jrow[c] = v[k][c];
-    }
-  }
-  if (tid == 0) {
-    perm[JJ] = p;
-    if (ipiv) ipiv[item * n + j0 + JJ] = j0 + p;
+        for (int c = JJ; c < NB; ++c) sm.row[buf][wid][c] = v[k][c];
+      }
+    sm.recip[buf][wid] = recipc(bv);
   }
   __syncthreads();
+  double wb[W];
+  int wp[W];
+#pragma unroll
+  for (int q = 0; q < W; ++q) {
+    wb[q] = sm.best[buf][q];
+    wp[q] = sm.place[buf][q];
+  }
+  best = wb[0];
+  int p = wp[0], w = 0;
+#pragma unroll
+  for (int q = 1; q < W; ++q) {  // (no branches: the loads go out together)
+    const bool more = (wb[q] > best) | ((wb[q] == best) & (wp[q] < p));
+    best = more ? wb[q] : best;
+    p = more ? wp[q] : p;
+    w = more ? q : w;
+  }
+  if (p >= pr) {  // NaN column: keep the diagonal
+    p = JJ;
+    w = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RPT; ++k)
+      if (pos[k] == JJ) {
+        sm.recip[buf][0] = recipc(v[k][JJ]);
+#pragma unroll
+        for (int c = JJ; c < NB; ++c) sm.row[buf][0][c] = v[k][c];
+      }
+    __syncthreads();
+  }
+  w = __builtin_amdgcn_readfirstlane(w);
+  const cd* prow = sm.row[buf][w];
   const cd piv = prow[JJ];
   const bool zero = (piv.x == 0.0 && piv.y == 0.0);
   if (zero && first_zero == 0) first_zero = j0 + JJ + 1;
-  const cd rp = zero ? mkc(0.0, 0.0) : recipc(piv);
+  const cd rp = zero ? mkc(0.0, 0.0) : sm.recip[buf][w];
+  if (tid == 0 && ipiv) ipiv[item * n + j0 + JJ] = j0 + p;
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
-    const int r = tid + k * TH;
-    if (r == JJ || r == p) {  // one set of loads: row JJ takes the pivot row, row p the old row JJ
-      const cd* src = (r == JJ) ? prow : jrow;
-#pragma unroll
-      for (int c = 0; c < NB; ++c) v[k][c] = src[c];
-    }
-    if (r > JJ && r < pr) {
-      const cd l = v[k][JJ] * rp;
+    pos[k] = pos[k] == p ? JJ : pos[k] == JJ ? p : pos[k];
+    if (pos[k] > JJ) {
+      // v rp with the second product rounded (written out: which of the two the
+      // compiler would round depends on the code around it)
+      const cd x = v[k][JJ];
+      const cd l = mkc(fma(x.x, rp.x, -(x.y * rp.y)), fma(x.x, rp.y, x.y * rp.x));
       v[k][JJ] = l;
 #pragma unroll
       for (int c = JJ + 1; c < NB; ++c) v[k][c] = fmsc(v[k][c], l, prow[c]);
@@ -552,28 +620,71 @@ __device__ __forceinline__ void panel_step(cd (&v)[RPT][NB], int nb, int pr, int
 }
 
 template <int NB, int RPT, int TH, int... J>
-__device__ __forceinline__ void panel_steps(std::integer_sequence<int, J...>, cd (&v)[RPT][NB], int nb, int pr, int j0,
-                                            int n, long long item, int* ipiv, int* perm, cd* prow, cd* jrow,
-                                            double* rv, int* ri, cd* rc, int& first_zero) {
-  (panel_step<NB, RPT, J, TH>(v, nb, pr, j0, n, item, ipiv, perm, prow, jrow, rv, ri, rc, first_zero), ...);
+__device__ __forceinline__ void panel_steps(std::integer_sequence<int, J...>, cd (&v)[RPT][NB], int (&pos)[RPT], int nb,
+                                            int pr, int j0, int n, long long item, int* ipiv, PanelLds<NB, TH>& sm,
+                                            int& first_zero) {
+  (panel_step<NB, RPT, J, TH>(v, pos, nb, pr, j0, n, item, ipiv, sm, first_zero), ...);
+}
+
+// After a register panel is factored: its interchanges on the other columns (and
+// B) and the triangular solve with L11, one thread per column.  The sixteen
+// interchanges as one permutation: the rows that end in the panel's first NB are
+// loaded at once, those that leave them are moved to where the former came from.
+template <int NB, int TH>
+__device__ __forceinline__ void panel_permute(int n, int m, int j0, int nb, cd* a, int lda, cd* bm, int ldb,
+                                              const cd* l11, const PanelLds<NB, TH>& sm, int keepL, int cend) {
+  const int nleft = (keepL & 1) ? j0 : 0;
+  const int nright = n - j0 - nb;
+  for (int e = threadIdx.x; e < nleft + nright + m; e += TH) {
+    const bool left = e < nleft, inA = e < nleft + nright;
+    cd* col = (left ? a + e : inA ? a + j0 + nb + (e - nleft) : bm + (e - nleft - nright)) +
+              (long long)j0 * (inA ? lda : ldb);
+    const long long ld = inA ? lda : ldb;
+    cd x[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) x[i] = (i < nb) ? col[sm.src[i] * ld] : mkc(0.0, 0.0);
+#pragma unroll
+    for (int g = 0; g < NB; g += 8) {
+      cd t[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t[i] = (g + i < nb && sm.dst[g + i] >= nb) ? col[(g + i) * ld] : mkc(0.0, 0.0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (g + i < nb && sm.dst[g + i] >= nb) col[sm.dst[g + i] * ld] = t[i];
+    }
+    const bool trsm = !left && (inA ? j0 + nb + (e - nleft) < cend : !(keepL & 2));
+    if (trsm) {
+#pragma unroll
+      for (int i = 1; i < NB; ++i)
+        if (i < nb) {
+#pragma unroll
+          for (int k = 0; k < i; ++k) x[i] = fmsc(x[i], l11[i * (NB + 1) + k], x[k]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if (i < nb && (trsm || sm.src[i] != i)) col[i * ld] = x[i];
+  }
 }
 
 // The same panel step with the panel in registers: thread t holds the
-// panel rows t, t + 256, .. (RPT of them, pr <= 256 RPT) and every pivot
-// step runs on registers, two barriers per column (the pivot search's
-// cross-wave reduction, then the exchange of rows jj and p through LDS,
-// which also broadcasts the pivot row).  Pivot choice, arithmetic and
-// output are those of zlu_panel_kernel: the largest |Re| + |Im| below the
-// diagonal, the first such row on ties, NaN columns keep the diagonal.
+// panel rows t, t + TH, .. (RPT of them, pr <= TH RPT) and every pivot
+// step runs on registers with one barrier.  Rows are not interchanged: each
+// thread follows its rows' places (which the first-row-on-ties rule needs) and
+// stores them there at the end.  Pivot choice, arithmetic and output are those
+// of zlu_panel_kernel: the largest |Re| + |Im| below the diagonal, the first such
+// row on ties, NaN columns keep the diagonal.
+// Bound by the latency of its steps (maximum, exchange, barrier, division) and of
+// the loads of the permuted columns.  With two barriers and a five-word shuffle
+// reduction per step and the interchanges in dependent groups of four, solves with
+// as many right-hand sides took (same results, bit for bit): n = 98, 40 systems (3
+// right-hand sides) 0.47 -> 0.34 ms, n = 162, 64: 1.00 -> 0.78, n = 242, 64: 1.71 ->
+// 1.38, n = 338, 24: 2.44 -> 1.90, n = 1 250, 8: 17.3 -> 15.3.
 template <int NB, int RPT, int TH = LB_THREADS>
 __global__ __launch_bounds__(TH, TH == 256 ? ((RPT == 1 && NB == 16) ? 4 : 2) : 1) void zlu_panel_reg_kernel(int n, int m, int j0, cd* A, int lda, long long sA,
                                                                    cd* B, int ldb, long long sB, int* ipiv, int* info,
                                                                    int keepL, int cend) {
-  __shared__ double rv[TH / 64];
-  __shared__ int ri[TH / 64];
-  __shared__ cd rc[TH / 64];
-  __shared__ int perm[NB];
-  __shared__ cd prow[NB], jrow[NB];
+  __shared__ PanelLds<NB, TH> sm;
   // L11 for the column solves, in dynamic LDS (NB (NB + 1) elements): with a
   // static array the compiler hoists all its loads out of the column loop
   extern __shared__ cd l11[];
@@ -585,31 +696,35 @@ __global__ __launch_bounds__(TH, TH == 256 ? ((RPT == 1 && NB == 16) ? 4 : 2) : 
   const int nb = min(NB, n - j0);
   const int pr = n - j0;
   cd v[RPT][NB];
+  int pos[RPT];
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
     const int r = tid + k * TH;
+    pos[k] = r < pr ? r : -1;
     const cd* src = a + (long long)(j0 + r) * lda + j0;
 #pragma unroll
     for (int c = 0; c < NB; ++c) v[k][c] = (r < pr && c < nb) ? src[c] : mkc(0.0, 0.0);
   }
-  panel_steps<NB, RPT, TH>(std::make_integer_sequence<int, NB>{}, v, nb, pr, j0, n, item, ipiv, perm, prow, jrow, rv, ri,
-                        rc, first_zero);
+  panel_steps<NB, RPT, TH>(std::make_integer_sequence<int, NB>{}, v, pos, nb, pr, j0, n, item, ipiv, sm, first_zero);
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
     const int r = tid + k * TH;
     if (r < pr) {
-      cd* dst = a + (long long)(j0 + r) * lda + j0;
+      cd* dst = a + (long long)(j0 + pos[k]) * lda + j0;
 #pragma unroll
       for (int c = 0; c < NB; ++c)
         if (c < nb) dst[c] = v[k][c];
-      if (r < NB) {
+      if (r < nb) sm.dst[r] = pos[k];
+      if (pos[k] < nb) {
+        sm.src[pos[k]] = r;
 #pragma unroll
-        for (int c = 0; c < NB; ++c) l11[r * (NB + 1) + c] = v[k][c];
+        for (int c = 0; c < NB; ++c) l11[pos[k] * (NB + 1) + c] = v[k][c];
       }
     }
   }
+  if (tid == 0 && info && (j0 == 0 || info[item] == 0)) info[item] = first_zero;
   __syncthreads();
-  panel_apply<NB, TH>(n, m, j0, nb, a, lda, bm, ldb, l11, NB + 1, perm, info, item, first_zero, keepL, cend);
+  panel_permute<NB, TH>(n, m, j0, nb, a, lda, bm, ldb, l11, sm, keepL, cend);
 }
 
 // X block = U11^-1 Y block for the rows j0 .. j0+nb of B (one thread per column)
@@ -834,9 +949,9 @@ static int launch_panel(hipStream_t s, int n, int m, int j0, Mat A, Mat B, int b
       else if (pr <= LB_THREADS)
         zlu_panel_reg_kernel<NB, 1><<<dim3(batch), dim3(LB_THREADS), l11, s>>>(n, m, j0, A.p, A.ld, A.stride, B.p,
                                                                               B.ld, B.stride, ipiv, info, mode, cend);
-      else if (pr <= 2 * LB_THREADS)
-        zlu_panel_reg_kernel<NB, 2><<<dim3(batch), dim3(LB_THREADS), l11, s>>>(n, m, j0, A.p, A.ld, A.stride, B.p,
-                                                                              B.ld, B.stride, ipiv, info, mode, cend);
+      else if (pr <= 512)
+        zlu_panel_reg_kernel<NB, 1, 512><<<dim3(batch), dim3(512), l11, s>>>(n, m, j0, A.p, A.ld, A.stride, B.p, B.ld,
+                                                                            B.stride, ipiv, info, mode, cend);
       else  // up to 1 536 rows: 512 threads, three rows each
         zlu_panel_reg_kernel<NB, 3, 512><<<dim3(batch), dim3(512), l11, s>>>(n, m, j0, A.p, A.ld, A.stride, B.p,
                                                                             B.ld, B.stride, ipiv, info, mode, cend);
