@@ -31,24 +31,21 @@ PEAK_FP64_TFLOPS = 78.6
 PEAK_HBM_GBS = 8000.0
 
 
-def eig_flops(n):
-    # Hessenberg + complex Schur + triangular eigenvectors: 110 n^3 real flops
-    # per matrix, minus the 4 n^3 back-transform W = Z X that runs as a GEMM.
-    return 106.0 * n ** 3
+def solve_flops(n, m):
+    """Real flops of one complex system of order n with m right-hand sides (complex
+    multiply-add = 8)."""
+    return 8 / 3 * n ** 3 + 8 * n * n * m
 
 
-def counted_flops_per_solve(n):
+def counted_flops_per_solve(n, doublings):
     """Real flops the library's own op sequence spends per disc_stack_bz solve (one unique
-    patterned layer, the R/T-only chain), complex multiply-add = 8 flops:
-    P Q (two N x N x n GEMMs) 4 n^3; eigensolver 106 n^3 and its
-    back-transform W = Z X 8 n^3; V = Q W (two GEMMs) 4 n^3; W^-1 from the
-    eigensolver's factors (one upper triangular solve with n right-hand sides
-    and one GEMM) 4 + 8 n^3; V^-1 V0 (LU + n right-hand sides) 8/3 + 8 n^3;
-    A^-1 (LU + n right-hand sides) and G2 = A^-1 B (one GEMM) 8/3 + 8 + 8 n^3;
-    T^-1 R2 (LU + 2n right-hand sides) 8/3 + 16 n^3; four n x n x n GEMMs
-    (X B G1, M B, M A, B G2) 32 n^3; the one chain junction (one GEMM, one LU,
-    vector solves) 11 n^3."""
-    return (4 + 106 + 8 + 4 + (4 + 8) + (8 / 3 + 8) + (8 / 3 + 8 + 8) + (8 / 3 + 16) + 32 + 11) * n ** 3
+    patterned layer, the R/T-only chain; `doublings` of its slice on average):
+    C^-1 T (N x N x n) 2 n^3; F^2 8; [F^3 | F^4] 16; F^4 U 16; C s (two N x N x n) 4;
+    s K C^-1 (n x N x N) 2; two systems of n right-hand sides each for the slice, every
+    doubling and the gap medium, two GEMMs per doubling 16; the one chain junction (one
+    GEMM 8, one system with one right-hand side)."""
+    return (2 + 8 + 16 + 16 + 4 + 2 + 16 * doublings + 8) * n ** 3 + 2 * (2 + doublings) * solve_flops(n, n) + \
+        solve_flops(n, 1)
 
 
 def cpu_info():
@@ -591,7 +588,7 @@ def run_autotune(step, args):
     return {"classes": len(table), "changed": changed, "mfma": mfma, "seconds": round(time.perf_counter() - t0, 2)}
 
 
-def load_traffic(kernel, workload, matrices_per_launch, avg_launch_ms):
+def load_traffic(kernel, workload, systems_per_launch, avg_launch_ms):
     """HBM bytes per launch from the committed FETCH_SIZE/WRITE_SIZE profile of
     the same workload and launch size (None when the profile does not match,
     or when the kernel's launch time moved by more than 5 % since, i.e. the
@@ -603,7 +600,7 @@ def load_traffic(kernel, workload, matrices_per_launch, avg_launch_ms):
         d = json.load(f)
     if d.get("workload") != workload:
         return None
-    if abs(d.get("matrices_per_launch", 0) - matrices_per_launch) > 0.01 * matrices_per_launch:
+    if abs(d.get("systems_per_launch", 0) - systems_per_launch) > 0.01 * systems_per_launch:
         return None
     ref_ms = d.get("avg_launch_ms")
     if ref_ms is None or abs(ref_ms - avg_launch_ms) > 0.05 * ref_ms:
@@ -694,18 +691,19 @@ def main():
     lib.khx_prof_enable(0)
     value = nsol * args.steps / el
 
-    # dominant kernel roofline: the eigen-solver (FP64, one matrix per workgroup)
-    eig_ms, eig_n = kern["zeig"]
-    avg_ms = eig_ms / max(eig_n, 1)
-    matrices_per_launch = nsol * args.steps / max(eig_n, 1)
-    flops_per_launch = eig_flops(n) * matrices_per_launch
-    achieved = flops_per_launch / (avg_ms * 1e-3) / 1e12
+    # dominant kernels roofline: the batched solve (FP64 matrix cores)
+    doublings = float(np.mean([np.mean(d.counts) for d in cl._plan.values()]))
+    lu_ms, lu_n = kern["zgesv_kernel"]
+    avg_ms = lu_ms / max(lu_n, 1)
+    per_solve = 2 * (2 + doublings) * solve_flops(n, n) + solve_flops(n, 1)
+    achieved = per_solve * nsol * args.steps / max(lu_ms * 1e-3, 1e-30) / 1e12
     workload = "disc_stack_bz pw(9,9) 65536 solves"
-    roofline = dict(bound="fp64", kernel="zeig (zeig_hess_kernel + zeig_qr_kernel + zeig_vec_kernel)", achieved=round(achieved, 4), peak=PEAK_FP64_TFLOPS,
-                    unit="TFLOP/s", frac=round(achieved / PEAK_FP64_TFLOPS, 6),
-                    traffic=load_traffic("zeig", workload, matrices_per_launch, avg_ms),
-                    avg_launch_ms=round(avg_ms, 4), matrices_per_launch=matrices_per_launch,
-                    flops_per_matrix=eig_flops(n))
+    systems_per_launch = (2 * (2 + doublings) + 1) * nsol * args.steps / max(lu_n, 1)
+    roofline = dict(bound="fp64", kernel="zgesv (gj_factor_kernel + gj_strips_kernel)", achieved=round(achieved, 4),
+                    peak=PEAK_FP64_TFLOPS, unit="TFLOP/s", frac=round(achieved / PEAK_FP64_TFLOPS, 6),
+                    traffic=load_traffic("zgesv", workload, systems_per_launch, avg_ms),
+                    avg_launch_ms=round(avg_ms, 4), systems_per_launch=round(systems_per_launch, 1),
+                    flops_per_solve=per_solve, doublings=round(doublings, 4))
     share = {k: round(v[0] / (el * 1e3 * 1.0), 4) for k, v in kern.items()}
 
     out = {
@@ -723,7 +721,7 @@ def main():
         pb = plain_batch1(cfg, idx, args.b1_sample)
         out["plain_fp64_batch1"] = pb
         out["speedup_vs_plain_batch1"] = round(out["value"] / pb["value"], 2)
-    cf = counted_flops_per_solve(n)
+    cf = counted_flops_per_solve(n, doublings)
     out["counted_flops"] = {"per_solve": cf, "tflops": round(value * cf / 1e12, 3),
                             "frac_fp64_peak": round(value * cf / 1e12 / PEAK_FP64_TFLOPS, 4),
                             "note": "the library's own op sequence (cheaper than the reference's, whose count is "
