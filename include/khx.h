@@ -123,7 +123,7 @@ int khx_convmat(const double* eps, int is_complex, int nx, int ny, int P, int Q,
 int khx_zgesv(int n, int nrhs, double* A, double* B, int batch, int* info, void* stream);
 
 /* The same with scratch (khx_zgesv_ws_bytes): blocked Gauss-Jordan on the
- * matrix cores in two launches for n <= 512, where A holds no LU factors
+ * matrix cores in few launches for n <= 512, where A holds no LU factors
  * afterwards; khx_zgesv beyond.                                            */
 size_t khx_zgesv_ws_bytes(int n, int batch);
 int khx_zgesv_ws(int n, int nrhs, double* A, double* B, int batch, int* info, void* ws, void* stream);

@@ -27,8 +27,8 @@
 // Work: 48 n^3 + 21 n^3 (slice) + 37 n^3 per doubling + 21 n^3 real operations,
 // all products and solves of full matrices, against a non-symmetric
 // eigenproblem whose bulge chase leaves the matrix cores idle.  Measured
-// through the eigensolver -> here: 24 layers of n = 338 167 -> 16.4 ms; 4 096
-// disc stacks of n = 162 415 -> 212 ms; the error against 64-bit references is
+// through the eigensolver -> here: 24 layers of n = 338 179 -> 8.5 ms; 4 096
+// disc stacks of n = 162 424 -> 103 ms; the error against 64-bit references is
 // the same or smaller (n = 50 against 80-bit arithmetic: 1e-14..1e-13 -> 2e-15..
 // 4e-14).
 #include "khx_internal.h"

@@ -153,7 +153,7 @@ def solve(A, B, overwrite_a=False, overwrite_b=False):
 
 
 def solve_conditioned(A, B, overwrite_a=False, overwrite_b=False):
-    """solve for well-conditioned systems (khx_zgesv_ws: two launches, Gauss-
+    """solve for well-conditioned systems (khx_zgesv_ws: few launches, Gauss-
     Jordan): the forward error is that of an LU, the residual of an
     ill-conditioned system may be larger."""
     lib = _lib.load()
