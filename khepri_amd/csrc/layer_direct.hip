@@ -81,13 +81,29 @@ dim3 grid_ew(long long total) {
 // ------------------------------------------------------------ |x| of a layer
 // Largest |eigenvalue| of F by power iteration, one workgroup per item, the
 // vector in LDS.  F v = J Q v + K C^-1 K^T (C v) needs three N x N matrix-vector
-// products and never forms F; a wavefront takes a row at a time (coalesced).
+// products and never forms F.  Sixteen lanes take a row, summed by DPP: a product
+// is one pass for N <= 32 and waits for one reduction of four steps (a wavefront
+// per row waited for six shuffles at every eighth row: a call with 1 item of N =
+// 25 83 -> 38 us, with 1 024 of N = 81 737 -> 175).
 // F is close to normal and its largest modes crowd near |K|^2 of the outermost
 // harmonics, where the start vector is concentrated: LAYER_POWER_STEPS steps
 // leave the estimate within a few per cent, and the approximant keeps full
 // precision that far above LAYER_THETA.
 constexpr int LAYER_POWER_STEPS = 8;
 constexpr int SCALE_THREADS = 512;
+
+// the sum over 16 lanes, in all of them
+__device__ __forceinline__ double row_sum16(double v) {
+#define KHX_ROR(n)                                                                            \
+  v += __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x120 + n, 0xf, 0xf, true), \
+                        __builtin_amdgcn_mov_dpp(__double2loint(v), 0x120 + n, 0xf, 0xf, true));
+  KHX_ROR(8)
+  KHX_ROR(4)
+  KHX_ROR(2)
+  KHX_ROR(1)
+#undef KHX_ROR
+  return v;
+}
 
 __global__ __launch_bounds__(SCALE_THREADS) void layer_scale_kernel(
     const cd* __restrict__ C, const cd* __restrict__ IC, long long cstride, const cd* __restrict__ kx,
@@ -102,7 +118,7 @@ __global__ __launch_bounds__(SCALE_THREADS) void layer_scale_kernel(
   const long long b = blockIdx.x;
   const cd* c = C + b * cstride;
   const cd* ic = IC + b * cstride;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, li = tid & 15;
   constexpr int NW = SCALE_THREADS / 64;
   for (int h = tid; h < N; h += SCALE_THREADS) {
     const cd x = kx[b * N + h], y = ky[b * N + h];
@@ -129,27 +145,27 @@ __global__ __launch_bounds__(SCALE_THREADS) void layer_scale_kernel(
   double n0 = norm2(v), best = 0.0;
   for (int it = 0; it < LAYER_POWER_STEPS; ++it) {
     const double sc = 1.0 / sqrt(n0);
-    for (int r = wid; r < N; r += NW) {
+    for (int r = tid >> 4; r < N; r += SCALE_THREADS / 16) {
       cd a1 = mkc(0.0, 0.0), a2 = mkc(0.0, 0.0);
-      for (int j = lane; j < N; j += 64) {
+      for (int j = li; j < N; j += 16) {
         const cd m = c[(long long)r * N + j];
         a1 = fmac(a1, m, v[j]);
         a2 = fmac(a2, m, v[N + j]);
       }
-      a1 = mkc(wave_sum(a1.x), wave_sum(a1.y));
-      a2 = mkc(wave_sum(a2.x), wave_sum(a2.y));
-      if (lane == 0) {
+      a1 = mkc(row_sum16(a1.x), row_sum16(a1.y));
+      a2 = mkc(row_sum16(a2.x), row_sum16(a2.y));
+      if (li == 0) {
         w[r] = a1;
         w[N + r] = a2;
         u[r] = fx[r] * a1 + fy[r] * a2;
       }
     }
     __syncthreads();
-    for (int r = wid; r < N; r += NW) {
+    for (int r = tid >> 4; r < N; r += SCALE_THREADS / 16) {
       cd a = mkc(0.0, 0.0);
-      for (int j = lane; j < N; j += 64) a = fmac(a, ic[(long long)r * N + j], u[j]);
-      a = mkc(wave_sum(a.x), wave_sum(a.y));
-      if (lane == 0) {
+      for (int j = li; j < N; j += 16) a = fmac(a, ic[(long long)r * N + j], u[j]);
+      a = mkc(row_sum16(a.x), row_sum16(a.y));
+      if (li == 0) {
         const cd x = fx[r], y = fy[r], t = y * v[r] - x * v[N + r];
         w[r] = sc * (x * a + y * t - w[r]);
         w[N + r] = sc * (y * a - x * t - w[N + r]);
