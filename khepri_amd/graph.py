@@ -41,12 +41,15 @@ def _same_plan(a, b):
 
 
 class _Captured:
+    sources = None   # kp, wl, te, tm on the device: the graph's own buffers, which every replay reads
+
     def __init__(self, crystal):
         self.cl = crystal
         self.batch = crystal.batch
 
     def _capture(self):
-        self.sources = tuple(t.clone() for t in self.cl._sources_dev)
+        if self.sources is None:   # (a later capture keeps them: update_sources has filled them)
+            self.sources = tuple(t.clone() for t in self.cl._sources_dev)
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):      # one warm-up on a side stream, as torch.cuda.graph expects
