@@ -30,6 +30,8 @@ gradient tensors are the graph's own buffers).
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import ops
@@ -56,7 +58,6 @@ class _Captured:
             with ops.deferred_status([]):
                 self._run()
         torch.cuda.current_stream().wait_stream(side)
-        self.plan = dict(self.cl._plan)
         self.graph = torch.cuda.CUDAGraph()
         self.status = []
         with torch.cuda.graph(self.graph):
@@ -65,11 +66,6 @@ class _Captured:
 
     def _run(self):
         raise NotImplementedError
-
-    def _planned(self):
-        cl = self.cl
-        layers = [cl.layers[name] for name in dict.fromkeys(cl.global_stacking)]
-        return plan_layers(layers, *self.sources[:2])
 
     def update_sources(self, wavelength, te=1.0, tm=1.0, theta=0.0, phi=0.0, kp=None):
         """New sources for the next replays (Crystal.set_source's arguments);
@@ -80,10 +76,6 @@ class _Captured:
             raise ValueError(f"the graph was captured for {self.batch} sources, got {cl.batch}")
         for dst, src in zip(self.sources, (cl._kp, cl._wl, cl._te, cl._tm)):
             dst.copy_(torch.as_tensor(src, device=dst.device))
-        # the captured launches are those of the layers' doubling counts, which
-        # the new sources may change: then the sequence is captured again
-        if not _same_plan(self._planned(), self.plan):
-            self._capture()
 
     def _replay(self, check):
         self.graph.replay()
@@ -100,6 +92,21 @@ class SolveGraph(_Captured):
         crystal.solve(rt_only=rt_only)       # eager: caches convolution matrices, tunes GEMM tiles
         crystal.poynting_flux_end()
         self._capture()
+
+    def _capture(self):
+        super()._capture()
+        self.plan = dict(self.cl._plan)
+
+    @functools.wraps(_Captured.update_sources)
+    def update_sources(self, *args, **kwargs):
+        super().update_sources(*args, **kwargs)
+        # the captured launches are those of the layers' doubling counts, which
+        # the new sources may change: then the sequence is captured again (a
+        # gradient's launches go through the modes and depend on no counts)
+        cl = self.cl
+        layers = [cl.layers[name] for name in dict.fromkeys(cl.global_stacking)]
+        if not _same_plan(plan_layers(layers, *self.sources[:2]), self.plan):
+            self._capture()
 
     def _run(self):
         cl = self.cl

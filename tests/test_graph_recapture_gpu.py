@@ -64,3 +64,30 @@ def test_solve_graph_after_an_eager_solve(gpu):
     for _ in range(2):
         for a, b in zip(g.replay(), ref.poynting_flux_end()):
             np.testing.assert_array_equal(a, b)
+
+
+def test_gradient_graph_is_captured_once(gpu):
+    """Its launches go through the modes: no new sources change them."""
+    from khepri_amd.graph import GradientGraph
+    cl = crystal((3, 3))
+    cl.set_source(WL, 1.0, 0.3)
+    g = GradientGraph(cl, wT=1.0)
+    graph, buffers = g.graph, g.outputs[2]["P"].data_ptr()
+    for src in (dict(kp=FAR), dict(kp=FAR), dict(theta=0.0)):
+        g.update_sources(WL, 1.0, 0.3, **src)
+        assert g.graph is graph and g.outputs[2]["P"].data_ptr() == buffers
+
+
+def test_solve_graph_is_captured_once_per_plan(gpu):
+    from khepri_amd.graph import SolveGraph
+    cl = crystal((3, 3))
+    cl.set_source(WL, 1.0, 0.3)
+    g = SolveGraph(cl)
+    graph = g.graph
+    g.update_sources(1.01 * WL, 1.0, 0.3)
+    assert g.graph is graph
+    g.update_sources(WL, 1.0, 0.3, kp=FAR)
+    graph2 = g.graph
+    assert graph2 is not graph
+    g.update_sources(1.01 * WL, 1.0, 0.3, kp=FAR)
+    assert g.graph is graph2
