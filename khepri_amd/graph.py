@@ -107,6 +107,7 @@ class SolveGraph(_Captured):
         layers = [cl.layers[name] for name in dict.fromkeys(cl.global_stacking)]
         if not _same_plan(plan_layers(layers, *self.sources[:2]), self.plan):
             self._capture()
+            cl.S = cl._RT = None   # the capture's: recorded, not computed (set_source left none)
 
     def _run(self):
         cl = self.cl

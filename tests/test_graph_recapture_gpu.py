@@ -91,3 +91,18 @@ def test_solve_graph_is_captured_once_per_plan(gpu):
     assert graph2 is not graph
     g.update_sources(1.01 * WL, 1.0, 0.3, kp=FAR)
     assert g.graph is graph2
+
+
+@pytest.mark.parametrize("rt_only", [None, True])
+def test_new_sources_leave_the_crystal_unsolved(gpu, rt_only):
+    """update_sources ran nothing for the crystal itself, recaptured or not: its
+    results, which a capture only records, cannot be read."""
+    from khepri_amd.graph import SolveGraph
+    cl = crystal((3, 3))
+    cl.set_source(WL, 1.0, 0.3)
+    g = SolveGraph(cl, rt_only=rt_only)
+    for src in (dict(theta=1.0), dict(kp=FAR)):
+        g.update_sources(WL, 1.0, 0.3, **src)
+        assert not cl.solved
+        with pytest.raises(AssertionError):
+            cl.poynting_flux_end()
