@@ -235,6 +235,8 @@ class Crystal:
             rt_only = (not want_reverse) and chunk < B
         if rt_only and want_reverse:
             raise ValueError("fields need the full S-matrix chain (rt_only=False)")
+        if B == 0 and not rt_only:
+            raise ValueError("the full S-matrix chain needs at least one source (rt_only=True takes none)")
         self.S = None
         self._RT = None
         if not torch.cuda.is_current_stream_capturing():   # a capture replays the plan of the call before it

@@ -255,7 +255,7 @@ int khx_zgesv_ws(int n, int nrhs, double* A, double* B, int batch, int* info, vo
 int khx_layer_scale(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
                     int batch, const double* k0d, double* est, void* stream) {
   KHX_ENTRY_BEGIN
-  KHX_REQUIRE(N > 0 && batch >= 0 && k0d && est, "khx_layer_scale: bad arguments");
+  KHX_REQUIRE(N > 0 && batch >= 0 && (batch == 0 || (k0d && est)), "khx_layer_scale: bad arguments");
   return khx::layer_scale(as_stream(stream), as_cd(C), as_cd(IC), per_item ? (long long)N * N : 0, as_cd(kx),
                           as_cd(ky), N, batch, k0d, est);
 }
@@ -267,7 +267,7 @@ size_t khx_layer_smatrix_ws_bytes(int n, int batch, int doublings) {
 int khx_layer_smatrix(const double* C, const double* IC, int per_item, const double* kx, const double* ky, int N,
                       int batch, const double* k0d, int doublings, double* S, int* info, void* ws, void* stream) {
   KHX_ENTRY_BEGIN
-  KHX_REQUIRE(N > 0 && batch >= 0 && k0d && S, "khx_layer_smatrix: bad arguments");
+  KHX_REQUIRE(N > 0 && batch >= 0 && (batch == 0 || (k0d && S && ws)), "khx_layer_smatrix: bad arguments");
   return khx::layer_smatrix(as_stream(stream), as_cd(C), as_cd(IC), per_item ? (long long)N * N : 0, as_cd(kx),
                             as_cd(ky), N, batch, k0d, doublings, as_cd(S), info, ws);
 }

@@ -282,7 +282,7 @@ def plan_layers(layers, kp, wl):
         planned = getattr(ly, "plan", None)
         if planned is not None:
             parts = [planned(kp[c:c + _PLAN_SOURCES], wl[c:c + _PLAN_SOURCES])
-                     for c in range(0, kp.shape[0], _PLAN_SOURCES)]
+                     for c in range(0, max(1, kp.shape[0]), _PLAN_SOURCES)]
             if parts[0] is not None:
                 est[id(ly)] = torch.cat(parts)
     if not est:
