@@ -52,7 +52,7 @@ class ExtendedLayer:
 
     def plan(self, kp, wl):
         """Layer.plan of the base at its own sources, (B Nb,) estimates."""
-        if not isinstance(self.base, Layer) or self.fields:
+        if getattr(type(self.base), "solve_batch", None) is not Layer.solve_batch or self.fields:
             return None
         kpb, wlb, _ = self._base_sources(kp, wl)
         self.base.fields = self.fields
@@ -75,7 +75,7 @@ class ExtendedLayer:
             self.W = self.V = self.L = None
             self.IC = 1.0
             return
-        self.base.solve_batch(kpb, wlb, doublings=doublings)
+        self.base.solve_batch(kpb, wlb, **({} if doublings is None else {"doublings": doublings}))
         self.info = getattr(self.base, "info", None)
         self.S = ops.joint_subspace(self.base.S, Nb, self.mode, 4)
         if self.fields:

@@ -181,8 +181,9 @@ class Layer:
         fuse = len(pat) >= 2 and B * len(pat) <= ops.eig_slots(2 * pat[0].expansion.N) and \
             all(ly.expansion is pat[0].expansion for ly in pat) and os.environ.get("KHX_FUSE_LAYERS", "1") == "1"
         if not fuse:
-            for ly in layers:
-                ly.solve_batch(kp, wl, rt_only=rt_only, doublings=plan.get(id(ly)))
+            for ly in layers:   # (a layer object of the caller's own need not know the argument)
+                known = {"doublings": plan[id(ly)]} if id(ly) in plan else {}
+                ly.solve_batch(kp, wl, rt_only=rt_only, **known)
             return
         dev = kp.device
         kx, ky = ops.kvectors(pat[0].expansion.g_device(dev), kp, wl)
@@ -274,14 +275,15 @@ def plan_layers(layers, kp, wl):
     """{id(layer): Doublings of its sources} for the layers of a stack whose
     S-matrices are formed without modes, over all sources of a solve: one
     estimate launch per layer and slice of sources, one host synchronisation
-    at the end (none between the chunks of the solve)."""
+    at the end (none between the chunks of the solve).  Only for the library's
+    own solve_batch: what another one does is not known here."""
+    from .extension import ExtendedLayer
     if ops.layer_route_is_modal():
         return {}
     est = {}
     for ly in layers:
-        planned = getattr(ly, "plan", None)
-        if planned is not None:
-            parts = [planned(kp[c:c + _PLAN_SOURCES], wl[c:c + _PLAN_SOURCES])
+        if getattr(type(ly), "solve_batch", None) in (Layer.solve_batch, ExtendedLayer.solve_batch):
+            parts = [ly.plan(kp[c:c + _PLAN_SOURCES], wl[c:c + _PLAN_SOURCES])
                      for c in range(0, max(1, kp.shape[0]), _PLAN_SOURCES)]
             if parts[0] is not None:
                 est[id(ly)] = torch.cat(parts)

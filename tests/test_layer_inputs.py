@@ -1,6 +1,57 @@
-"""Layers and batches that the chain takes beside its own solved layers."""
+"""Layers and batches that the chain takes beside its own solved layers: objects
+with the layer protocol, subclasses, hand-made S-matrices, empty batches."""
 import numpy as np
 import pytest
+import torch
+
+
+class Own:
+    """The protocol of Crystal.add_layer: solve_batch(kp, wl, ws, rt_only)."""
+    depth, fields, S = 0.3, False, None
+
+    def solve_batch(self, kp, wl, ws=None, rt_only=False):
+        self.S = (kp, wl, rt_only)
+
+
+def test_layer_objects_with_the_plain_protocol():
+    from khepri_amd.layer import Layer, plan_layers
+    kp, wl = torch.zeros((2, 2), dtype=torch.complex128), torch.ones(2, dtype=torch.float64)
+    ly = Own()
+    assert plan_layers([ly], kp, wl) == {}
+    Layer.solve_batch_many([ly], kp, wl, rt_only=True)
+    assert ly.S[2] is True
+
+
+def test_subclass_with_its_own_solve_batch():
+    """Its solve decides what becomes of the S-matrix: nothing is planned for it."""
+    from khepri_amd import Crystal
+    from khepri_amd.layer import Layer, plan_layers
+
+    class Sub(Layer):
+        def solve_batch(self, kp, wl, ws=None, rt_only=False):
+            self.S = kp
+    kp, wl = torch.zeros((2, 2), dtype=torch.complex128), torch.ones(2, dtype=torch.float64)
+    ly = Sub.pixmap(Crystal((1, 1)).expansion, np.eye(8) + 1.0, 0.3)
+    assert plan_layers([ly], kp, wl) == {}
+    Layer.solve_batch_many([ly], kp, wl)
+    assert ly.S is kp
+
+
+def test_extended_layer_over_such_a_base():
+    from khepri_amd.extension import ExtendedLayer
+    from khepri_amd.layer import Layer
+
+    class Sub(Layer):
+        def solve_batch(self, kp, wl, ws=None, rt_only=False):
+            raise StopIteration                    # reached with the plain arguments
+    base = Sub()
+    base.formulation, base.expansion = 1, None
+    ext = ExtendedLayer.__new__(ExtendedLayer)
+    ext.__dict__.update(base=base, fields=False, mode=0, gs=np.zeros((2, 1)))
+    kp, wl = torch.zeros((2, 2), dtype=torch.complex128), torch.ones(2, dtype=torch.float64)
+    assert ext.plan(kp, wl) is None
+    with pytest.raises(StopIteration):
+        ext.solve_batch(kp, wl)
 
 
 @pytest.mark.gpu
