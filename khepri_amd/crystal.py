@@ -246,7 +246,7 @@ class Crystal:
             self._check_layers(names)
             infos = []
             self.stacking_matrices, self.stacking_reverse_matrices, self.Stot = stack_layers(
-                self.expansion.pw, stacked, self.stack_retain_mask, reverse=want_reverse, infos=infos)
+                self.expansion.pw, stacked, self.stack_retain_mask, reverse=want_reverse, infos=infos, solved=True)
             for info in infos:
                 self._check_info(info, "star product", lu=True)
             self.S = self.Stot
@@ -291,7 +291,7 @@ class Crystal:
         else:
             infos = []
             _, _, Stot = stack_layers(self.expansion.pw, stacked, self.stack_retain_mask, reverse=False,
-                                      infos=infos)
+                                      infos=infos, solved=True)
             for info in infos:
                 self._check_info(info, "star product", lu=True)
             r, t, ro, to = ops.poynting(Stot, g, kp, wl, te_all[sl], tm_all[sl], self.epsi, self.epse,

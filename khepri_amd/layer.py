@@ -158,7 +158,7 @@ class Layer:
     def structure(self):
         """("identity", None) for a half space of the gap medium, ("prop", X) for
         a uniform layer of it (X its propagation factors), else ("dense", S):
-        what a star product with this layer amounts to."""
+        what a star product with this layer, as solve_batch left it, amounts to."""
         if np.isscalar(self.epsilon) and complex(self.epsilon) == 1:
             if self.formulation in (Formulation.HALF_SPACE_INC, Formulation.HALF_SPACE_TRN):
                 return ("identity", None)
@@ -307,7 +307,8 @@ def scattering_identity(B, n, device):
 def _stack_forward(layers, ws, infos):
     """Total S-matrix from each layer's structure; None when no layer is dense."""
     from . import chain
-    seq = chain.dense_sequence([ly.structure() if isinstance(ly, Layer) else ("dense", ly.S) for ly in layers])
+    own = [getattr(type(ly), "solve_batch", None) is Layer.solve_batch for ly in layers]
+    seq = chain.dense_sequence([ly.structure() if o else ("dense", ly.S) for o, ly in zip(own, layers)])
     if len(layers) < 2 or isinstance(seq, tuple) or not seq:
         return None
     Stot = seq[0]
@@ -318,7 +319,7 @@ def _stack_forward(layers, ws, infos):
     return Stot
 
 
-def stack_layers(pw, layers, mask, reverse=True, ws=None, infos=None):
+def stack_layers(pw, layers, mask, reverse=True, ws=None, infos=None, solved=False):
     """Forward chain S_I * S_0 * S_1 * ... (copies kept where mask) and the
     reverse chain (khepri/layer.py:35-60).
 
@@ -326,12 +327,13 @@ def stack_layers(pw, layers, mask, reverse=True, ws=None, infos=None):
     formed.  The reverse chain is only needed for fields (``reverse=False``
     skips it and returns None for it).  ``infos``, when a list, receives the
     device status word of every star product (first zero pivot of D or F,
-    where the reference's numpy solve raises LinAlgError).  Without fields
+    where the reference's numpy solve raises LinAlgError).  solved: the layers'
+    S-matrices are what their solve_batch has just left.  Then, without fields
     and inner copies, layers of the gap medium are not multiplied: its half
     spaces are the identity, its uniform layers diagonal scalings of a
     neighbour (a third of the star products of a typical stack are left).
     """
-    if not reverse and not any(mask[1:-1]):
+    if solved and not reverse and not any(mask[1:-1]):
         Stot = _stack_forward(layers, ws, infos)
         if Stot is not None:
             return [layers[0].S if mask[0] else None, *[None] * (len(layers) - 2), Stot if mask[-1] else None], \

@@ -54,6 +54,53 @@ def test_extended_layer_over_such_a_base():
         ext.solve_batch(kp, wl)
 
 
+def _recorded(monkeypatch):
+    """ops.redheffer replaced by a record of its operands."""
+    from khepri_amd import ops
+    seen = []
+
+    def redheffer(SA, SB, ws=None, gj=False):
+        seen.append((SA, SB))
+        return SA, None
+    monkeypatch.setattr(ops, "redheffer", redheffer)
+    return seen
+
+
+def test_stack_layers_reads_the_given_s(monkeypatch):
+    """stack_layers multiplies the S-matrices that its layers hold, whatever their
+    permittivity says and also where a layer has none."""
+    from khepri_amd import Crystal
+    from khepri_amd.layer import Layer, stack_layers
+    e = Crystal((1, 1)).expansion
+    seen = _recorded(monkeypatch)
+    layers = [Layer(), Layer.half_infinite(e, "reflexion", 1), Layer.uniform(e, 1, 0.3), Layer.uniform(e, 2.0, 0.3)]
+    for k, ly in enumerate(layers):
+        ly.S = torch.full((1, 2, 2, 2, 2), k, dtype=torch.complex128)
+    layers[2].X = torch.ones((1, 2), dtype=torch.complex128)   # of an earlier solve
+    stack_layers(None, layers, [True, False, False, True], reverse=False)
+    assert [id(b) for _, b in seen] == [id(ly.S) for ly in layers[1:]]
+    assert seen[0][0] is layers[0].S
+
+
+def test_fold_is_for_layers_as_solved_by_the_library(monkeypatch):
+    """Where the stack was just solved, gap-medium layers fold; those of another solve_batch do not."""
+    from khepri_amd import Crystal
+    from khepri_amd.layer import Layer, stack_layers
+
+    class Sub(Layer):
+        def solve_batch(self, kp, wl, ws=None, rt_only=False):
+            super().solve_batch(kp, wl, ws, rt_only)
+    e = Crystal((1, 1)).expansion
+    for kind, products in ((Layer, 0), (Sub, 1)):
+        seen = _recorded(monkeypatch)
+        layers = [kind.half_infinite(e, "reflexion", 1), Layer.uniform(e, 2.0, 0.3)]
+        for ly in layers:
+            ly.S = torch.zeros((1, 2, 2, 2, 2), dtype=torch.complex128)
+        Stot = stack_layers(None, layers, [True, True], reverse=False, solved=True)[2]
+        assert len(seen) == products
+        assert Stot is (layers[1].S if products == 0 else layers[0].S)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["pixmap", "uniform"])
 def test_empty_batch(gpu, kind):
