@@ -193,9 +193,9 @@ int khx_patterned_layer_cached(const double* C, const double* IC, int per_item, 
  * layer cut into 2^doublings slices, then as many star products of a slab with
  * itself.
  * khx_layer_scale: est[b] = |k0d sqrt(eigenvalue of P Q)| / 2 of the largest
- *   eigenvalue, by power iteration (a few per cent; NaN for a non-finite
- *   input).  The approximant is exact to FP64 rounding while
- *   est / 2^doublings <= KHX_LAYER_THETA, so
+ *   eigenvalue, by power iteration (at least 0.87 of the true value in 20 000
+ *   drawn maps; NaN for a non-finite input).  The approximant is exact to FP64
+ *   rounding up to 4.7 and KHX_LAYER_THETA leaves room for such an estimate:
  *   doublings = max(0, ceil(log2(est / KHX_LAYER_THETA))).
  * khx_layer_smatrix: S (batch, 2, 2, n, n), one number of doublings for the
  *   whole batch.  info[b]: 1 a non-finite entry in P Q (numpy's eig raises),

@@ -85,11 +85,18 @@ dim3 grid_ew(long long total) {
 // is one pass for N <= 32 and waits for one reduction of four steps (a wavefront
 // per row waited for six shuffles at every eighth row: a call with 1 item of N =
 // 25 83 -> 38 us, with 1 024 of N = 81 737 -> 175).
-// F is close to normal and its largest modes crowd near |K|^2 of the outermost
-// harmonics, where the start vector is concentrated: LAYER_POWER_STEPS steps
-// leave the estimate within a few per cent, and the approximant keeps full
-// precision that far above LAYER_THETA.
+// One step's growth |F v| / |v| approaches the largest |eigenvalue| from below
+// where F is close to normal (its largest modes crowd near |K|^2 of the outermost
+// harmonics, where the start vector is concentrated).  Where the permittivity
+// changes sign they come in pairs of nearly opposite sign, and one step grows as
+// much as the next shrinks: the estimate is the largest of the last step's growth
+// and the geometric means over the last 2 to LAYER_POWER_MEANS steps.  Against
+// eigenvalues from numpy, 20 000 drawn maps: at least 0.87 of the true |x| (0.89
+// without sign changes and metals; the last step alone: 0.50), up to 2.3 times it
+// where the sign changes, 1.04 elsewhere.  So a slice has |x| <= 4 / 0.87 = 4.6,
+// where the approximant's error is 6e-17 (1e-16 at 4.7, 1e-15 at 5, 4e-13 at 6).
 constexpr int LAYER_POWER_STEPS = 8;
+constexpr int LAYER_POWER_MEANS = 6;
 constexpr int SCALE_THREADS = 512;
 
 // the sum over 16 lanes, in all of them
@@ -114,7 +121,7 @@ __global__ __launch_bounds__(SCALE_THREADS) void layer_scale_kernel(
   cd* u = sm + 4 * N;   // N
   cd* fx = sm + 5 * N;  // kx
   cd* fy = sm + 6 * N;  // ky
-  __shared__ double red[SCALE_THREADS / 64];
+  __shared__ double red[SCALE_THREADS / 64], growth[LAYER_POWER_STEPS];  // growth: thread 0's
   const long long b = blockIdx.x;
   const cd* c = C + b * cstride;
   const cd* ic = IC + b * cstride;
@@ -142,7 +149,7 @@ __global__ __launch_bounds__(SCALE_THREADS) void layer_scale_kernel(
     __syncthreads();
     return t;
   };
-  double n0 = norm2(v), best = 0.0;
+  double n0 = norm2(v);
   for (int it = 0; it < LAYER_POWER_STEPS; ++it) {
     const double sc = 1.0 / sqrt(n0);
     for (int r = tid >> 4; r < N; r += SCALE_THREADS / 16) {
@@ -175,9 +182,23 @@ __global__ __launch_bounds__(SCALE_THREADS) void layer_scale_kernel(
     for (int h = tid; h < 2 * N; h += SCALE_THREADS) v[h] = w[h];
     __syncthreads();
     n0 = norm2(v);  // = |F v|^2 / |v|^2 of this step
-    best = n0;
+    if (tid == 0) growth[it] = n0;
   }
-  if (tid == 0) est[b] = 0.5 * fabs(k0d[b]) * sqrt(sqrt(best));
+  if (tid == 0) {
+    bool shrank = false;  // no mean exceeds the last step otherwise
+#pragma unroll
+    for (int w = 2; w <= LAYER_POWER_MEANS; ++w) shrank |= growth[LAYER_POWER_STEPS - w] > n0;
+    double best = n0;
+    if (shrank) {
+      double sum = log2(n0);
+      for (int w = 2; w <= LAYER_POWER_MEANS; ++w) {
+        sum += log2(growth[LAYER_POWER_STEPS - w]);
+        const double mean = exp2(sum / w);
+        if (mean > best) best = mean;
+      }
+    }
+    est[b] = 0.5 * fabs(k0d[b]) * sqrt(sqrt(best));
+  }
 }
 
 // ------------------------------------------------------------ F
