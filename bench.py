@@ -581,7 +581,7 @@ def run_autotune(step, args):
     from khepri_amd import autotune
     t0 = time.perf_counter()
     table = autotune.autotune(step)
-    changed = sum(1 for e in table.values() if e["tile"] != autotune.default_tile(*e["shape"][:2]))
+    changed = sum(1 for e in table.values() if e["tile"] != autotune.library_tile(*e["shape"][:2], e["shape"][5]))
     mfma = sum(1 for e in table.values() if e["tile"] >= 4)
     print(f"[bench] gemm autotune: {len(table)} classes, {changed} changed, {mfma} on MFMA", file=sys.stderr,
           flush=True)

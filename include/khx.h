@@ -409,9 +409,11 @@ int khx_eig_slots(int n);
  * records of 6 ints (M, N, K, opA, opB, batch) into shapes, returning the
  * count.  khx_gemm_force(cfg) uses tile cfg for every GEMM (-1: off);
  * khx_gemm_tune_set installs the choice for one shape class (batch is
- * bucketed: < 16, < 256, >= 256; cfg -1 removes it).                       */
+ * bucketed: < 16, < 256, >= 256; cfg -1 removes it); khx_gemm_default_tile
+ * is the library's choice where none is installed.                         */
 int khx_gemm_record(int on, int* shapes, int max_shapes);
 int khx_gemm_force(int cfg);
+int khx_gemm_default_tile(int M, int N, int batch);
 int khx_gemm_tune_set(int M, int N, int K, int opa, int opb, int batch, int cfg);
 
 /* Measurement support (no counterpart in the reference).

@@ -94,6 +94,7 @@ SIGNATURES = {
     "khx_eig_slots": (_i, [_i]),
     "khx_gemm_record": (_i, [_i, _vp, _i]),
     "khx_gemm_force": (_i, [_i]),
+    "khx_gemm_default_tile": (_i, [_i, _i, _i]),
     "khx_gemm_tune_set": (_i, [_i, _i, _i, _i, _i, _i, _i]),
     "khx_prof_enable": (_i, [_i]),
     "khx_prof_collect": (_i, [C.c_char_p, C.POINTER(C.c_double), C.POINTER(C.c_longlong)]),

@@ -4,8 +4,8 @@ libkhx's zgemm comes in eight kernels of 256 threads: FP64 FMA register
 tiles (M x N per workgroup) 0 = 64x64, 1 = 32x32, 2 = 64x32, 3 = 32x64, and
 the same tiles on the FP64 matrix cores (v_mfma_f64_16x16x4f64) 4 = 64x64,
 5 = 32x32, 6 = 64x32, 7 = 32x64.  Without a tuning table the library takes
-MFMA 32x32 when either side is at most 96 and MFMA 32x64 otherwise
-(``default_tile``).  The tuner
+MFMA 32x32, or MFMA 64x64 for many tiles of a large product
+(``library_tile``).  The tuner
 
 1. runs a workload once with shape recording on (``record``), which collects
    every distinct (M, N, K, opA, opB, batch) the library launches;
@@ -40,8 +40,17 @@ _OPNAME = {0: "N", 1: "T", 2: "C"}
 
 
 def default_tile(M, N):
-    """The library's choice for an (M x N) product when no table entry applies."""
+    """A rule by the sides alone (MFMA 32x32 up to 96, else 32x64).  What the library
+    takes when no table entry applies is library_tile."""
     return 5 if min(M, N) <= 96 else 7
+
+
+def library_tile(M, N, batch):
+    """The library's choice for `batch` (M x N) products when no table entry applies."""
+    tile = _lib.load().khx_gemm_default_tile(M, N, batch)
+    if tile < 0:
+        check(tile, "khx_gemm_default_tile")
+    return tile
 
 
 def _bucket(batch):

@@ -497,6 +497,11 @@ unsigned long long tune_key(int M, int N, int K, int oa, int ob, int batch) {
 }
 }  // namespace
 
+int gemm_default_tile(int M, int N, int batch) {
+  const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
+  return M >= 1024 && N >= 1024 && tiles64 >= 2048 ? 4 : 5;
+}
+
 int gemm_tile_choice(int M, int N, int K, int oa, int ob, int batch) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   if (g_force >= 0) return g_force;
@@ -509,8 +514,7 @@ int gemm_tile_choice(int M, int N, int K, int oa, int ob, int batch) {
   }
   const auto it = g_tune.find(key);
   if (it != g_tune.end()) return it->second;
-  const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64) * batch;
-  return M >= 1024 && N >= 1024 && tiles64 >= 2048 ? 4 : 5;
+  return gemm_default_tile(M, N, batch);
 }
 
 template <int OA, int OB>

@@ -479,6 +479,12 @@ int khx_gemm_force(int cfg) {
   return khx::gemm_force(cfg);
 }
 
+int khx_gemm_default_tile(int M, int N, int batch) {
+  KHX_ENTRY_BEGIN
+  KHX_REQUIRE(M > 0 && N > 0 && batch > 0, "khx_gemm_default_tile: bad shape");
+  return khx::gemm_default_tile(M, N, batch);
+}
+
 int khx_gemm_tune_set(int M, int N, int K, int opa, int opb, int batch, int cfg) {
   KHX_ENTRY_BEGIN
   KHX_REQUIRE(M > 0 && N > 0 && K > 0 && opa >= 0 && opa <= 2 && opb >= 0 && opb <= 2 && batch > 0,

@@ -26,6 +26,7 @@ int zgemm_op(hipStream_t s, int opa, int opb, int M, int N, int K, cd alpha, Mat
 // GEMM tile selection (tuning table, forced choice, shape recording)
 int gemm_tune_set(int M, int N, int K, int oa, int ob, int batch, int cfg);
 int gemm_force(int cfg);
+int gemm_default_tile(int M, int N, int batch);
 int gemm_record(int on, int* shapes, int max_shapes);
 // Solve A X = B (A n x n destroyed, B n x m overwritten); info[b] = first zero pivot (1-based) or 0
 int zgesv(hipStream_t s, int n, int m, Mat A, Mat B, int batch, int* info);
