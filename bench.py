@@ -588,6 +588,42 @@ def run_autotune(step, args):
     return {"classes": len(table), "changed": changed, "mfma": mfma, "seconds": round(time.perf_counter() - t0, 2)}
 
 
+def plan_doublings(plan):
+    """Mean doublings over the layers of a solve's plan (Crystal._plan); None where the
+    counted sequence is not the one that ran: no plan (S-matrices through the
+    eigensolver, KHX_LAYER_MODES=1 or a switch of that path) or items of count -1."""
+    counts = [d.counts for d in plan.values()]
+    if not counts or min(c.min() for c in counts) < 0:
+        return None
+    return float(np.mean([np.mean(c) for c in counts]))
+
+
+def solve_roofline(doublings, n, nsol, steps, lu_ms, lu_n, workload):
+    """Roofline of the dominant kernels, the batched solve (FP64 matrix cores), from its
+    measured time; None without counted doublings."""
+    if doublings is None:
+        return None
+    avg_ms = lu_ms / max(lu_n, 1)
+    per_solve = 2 * (2 + doublings) * solve_flops(n, n) + solve_flops(n, 1)
+    achieved = per_solve * nsol * steps / max(lu_ms * 1e-3, 1e-30) / 1e12
+    systems_per_launch = (2 * (2 + doublings) + 1) * nsol * steps / max(lu_n, 1)
+    return dict(bound="fp64", kernel="zgesv (gj_factor_kernel + gj_strips_kernel)", achieved=round(achieved, 4),
+                peak=PEAK_FP64_TFLOPS, unit="TFLOP/s", frac=round(achieved / PEAK_FP64_TFLOPS, 6),
+                traffic=load_traffic("zgesv", workload, systems_per_launch, avg_ms),
+                avg_launch_ms=round(avg_ms, 4), systems_per_launch=round(systems_per_launch, 1),
+                flops_per_solve=per_solve, doublings=round(doublings, 4))
+
+
+def counted_line(doublings, n, value):
+    """The counted operations of the whole sequence at `value` solves/s; None as solve_roofline."""
+    if doublings is None:
+        return None
+    cf = counted_flops_per_solve(n, doublings)
+    return {"per_solve": cf, "tflops": round(value * cf / 1e12, 3),
+            "frac_fp64_peak": round(value * cf / 1e12 / PEAK_FP64_TFLOPS, 4),
+            "note": "the library's own op sequence (cheaper than the reference's, whose count is 2.578e9 per solve)"}
+
+
 def load_traffic(kernel, workload, systems_per_launch, avg_launch_ms):
     """HBM bytes per launch from the committed FETCH_SIZE/WRITE_SIZE profile of
     the same workload and launch size (None when the profile does not match,
@@ -691,19 +727,9 @@ def main():
     lib.khx_prof_enable(0)
     value = nsol * args.steps / el
 
-    # dominant kernels roofline: the batched solve (FP64 matrix cores)
-    doublings = float(np.mean([np.mean(d.counts) for d in cl._plan.values()]))
-    lu_ms, lu_n = kern["zgesv_kernel"]
-    avg_ms = lu_ms / max(lu_n, 1)
-    per_solve = 2 * (2 + doublings) * solve_flops(n, n) + solve_flops(n, 1)
-    achieved = per_solve * nsol * args.steps / max(lu_ms * 1e-3, 1e-30) / 1e12
+    doublings = plan_doublings(cl._plan)
     workload = "disc_stack_bz pw(9,9) 65536 solves"
-    systems_per_launch = (2 * (2 + doublings) + 1) * nsol * args.steps / max(lu_n, 1)
-    roofline = dict(bound="fp64", kernel="zgesv (gj_factor_kernel + gj_strips_kernel)", achieved=round(achieved, 4),
-                    peak=PEAK_FP64_TFLOPS, unit="TFLOP/s", frac=round(achieved / PEAK_FP64_TFLOPS, 6),
-                    traffic=load_traffic("zgesv", workload, systems_per_launch, avg_ms),
-                    avg_launch_ms=round(avg_ms, 4), systems_per_launch=round(systems_per_launch, 1),
-                    flops_per_solve=per_solve, doublings=round(doublings, 4))
+    roofline = solve_roofline(doublings, n, nsol, args.steps, *kern["zgesv_kernel"], workload)
     share = {k: round(v[0] / (el * 1e3 * 1.0), 4) for k, v in kern.items()}
 
     out = {
@@ -721,11 +747,7 @@ def main():
         pb = plain_batch1(cfg, idx, args.b1_sample)
         out["plain_fp64_batch1"] = pb
         out["speedup_vs_plain_batch1"] = round(out["value"] / pb["value"], 2)
-    cf = counted_flops_per_solve(n, doublings)
-    out["counted_flops"] = {"per_solve": cf, "tflops": round(value * cf / 1e12, 3),
-                            "frac_fp64_peak": round(value * cf / 1e12 / PEAK_FP64_TFLOPS, 4),
-                            "note": "the library's own op sequence (cheaper than the reference's, whose count is "
-                                    "2.578e9 per solve)"}
+    out["counted_flops"] = counted_line(doublings, n, value)
     if args.grad_steps > 0:
         out["grad_grid"] = grad_grid_rate(args.grad_steps)
         print("[bench] grad_grid done", file=sys.stderr, flush=True)
