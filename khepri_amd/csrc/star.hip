@@ -51,13 +51,15 @@ size_t star_ws_bytes(int n, int batch) {
   return (size_t)8 * n * n * sizeof(cd) * batch + (size_t)2 * (n + 1) * batch * sizeof(int) + 256;
 }
 
-// gj: one solve, through the Gauss-Jordan (zgesv_ws; D is well conditioned for
-// passive layers): a pass with one product of order 1 250 for 8 sources 48.4 -> 40.3
-// ms against two solves, 151 products of order 50 0.10 ms less.  The chains that
-// fields or gradients are read from keep the LU: the mode amplitudes inside a
-// layer are differences of terms as large as e^{lambda d}, the eigenvector
-// adjoint divides by mode differences, and both carry every rounding of the chain
-// magnified as much.
+// gj: one solve, through the Gauss-Jordan (zgesv_ws).  Near a pole of a layer's
+// S-matrix against the gap D is ill conditioned; R and T are then as near as with
+// two LU solves (155 stacks on such poles against 80-bit arithmetic, lu_gj.hip: mean
+// of the logarithm 3.6e-13, with LU 3.1e-13, modes and two LU solves 3.7e-13).  A
+// pass with one product of order 1 250 for 8 sources 48.4 -> 40.3 ms against two
+// solves, 151 products of order 50 0.10 ms less.  The chains that fields or
+// gradients are read from keep the LU: the mode amplitudes inside a layer are
+// differences of terms as large as e^{lambda d}, the eigenvector adjoint divides by
+// mode differences, and both carry every rounding of the chain magnified as much.
 int star(hipStream_t s, const cd* SA, long long sA, const cd* SB, long long sB, int n, int batch, cd* S,
          int* info, void* wsv, bool gj) {
   if (batch <= 0) return 0;

@@ -153,9 +153,9 @@ def solve(A, B, overwrite_a=False, overwrite_b=False):
 
 
 def solve_conditioned(A, B, overwrite_a=False, overwrite_b=False):
-    """solve for well-conditioned systems (khx_zgesv_ws: few launches, Gauss-
-    Jordan): the forward error is that of an LU, the residual of an
-    ill-conditioned system may be larger."""
+    """solve where only X is wanted, to the forward error of an LU (khx_zgesv_ws: few
+    launches, Gauss-Jordan); the residual of an ill-conditioned system may be
+    larger than an LU's."""
     lib = _lib.load()
     Af = _owned(A, overwrite_a)
     X = _owned(B, overwrite_b)
@@ -404,8 +404,9 @@ def _layer_smatrix(C, IC, kx, ky, k0d, doublings, S, info):
 def layer_smatrix(C, IC, kx, ky, k0d, doublings):
     """(S (B, 2, 2, n, n), status words) of a patterned layer without its
     modes; doublings: the items' Doublings.  The items of one count
-    are solved together, so an item's result does not depend on the batch it
-    comes in."""
+    are solved together, so an item gets the same doublings in whatever batch it
+    comes; the products and solves choose their tiles by the batch, so its result
+    is the same to rounding (to the bit where the choice does not change)."""
     B, N = kx.shape
     n = 2 * N
     dev = kx.device
