@@ -39,7 +39,9 @@ class CrystalBatch:
         self.device = torch.device(device) if device is not None else None
         env = os.environ.get("KHX_BATCH_CHUNK")
         # patterned layers per launch; default: the eigensolver's resident
-        # slots at the group's order, so every launch is one full round
+        # slots at the group's order, so every launch with modes is one full
+        # round (without, 1 024 devices: 1 622 devices/s, 1 515 in launches of
+        # 256, 1 665 of 2 048)
         self.chunk = chunk or (int(env) if env else None)
 
     def _dev(self):

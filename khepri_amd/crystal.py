@@ -192,7 +192,9 @@ class Crystal:
         chunk = int(max(1, min(B, budget // per)))
         if chunk < B and self._has_patterned():
             # every chunk's eigensolver launch is a whole number of rounds of
-            # resident workgroups: a partly filled last round costs a full one
+            # resident workgroups: a partly filled last round costs a full one.
+            # (Without modes the size matters little: 16 384 solves at 81 harmonics
+            # in chunks of 512, 1 024, 2 048: 32 260, 32 550, 32 440 solves/s.)
             slots = ops.eig_slots(n)
             if chunk >= slots:
                 chunk = chunk // slots * slots

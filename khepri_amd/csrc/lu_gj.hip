@@ -29,10 +29,11 @@
 // updates and 22 leaf launches for n = 162 and moves the trailing matrix once per
 // panel.  Measured, LU -> here, ms: n = 50 (50 right-hand sides) 2 systems 0.28 ->
 // 0.055, 4 096 systems 4.4 -> 0.37; n = 162 (162) 2 048 systems 7.0 -> 3.55; n =
-// 338 (338) 512 systems 11.1 -> 6.8, 2 systems 0.72.  The solve runs at about 70 %
-// of the FP64 matrix rate; the factorization is bound by the latency of its pivot
-// steps (0.6 to 0.9 us: the updates and keys of 16 registers 0.25, candidates,
-// barrier and winner 0.2, reciprocal 0.1) and of a panel's loads and products.
+// 338 (338) 512 systems 11.1 -> 6.8, 2 systems 0.72.  The strips keep the FP64
+// matrix pipe 67 % busy (n = 162, 2 048 systems), the factorization 31 %: it is
+// bound by the latency of its pivot steps (0.6 to 0.9 us: the updates and keys of 16
+// registers 0.25, candidates, barrier and winner 0.2, reciprocal 0.1) and of a
+// panel's loads and products.
 // Error: forward error as an LU's; the residual of an ill-conditioned system can
 // be larger (Gauss-Jordan is not row-wise backward stable).  Most systems it serves
 // are well conditioned (the slice and the doublings, formed against a medium in

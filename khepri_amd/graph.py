@@ -20,8 +20,9 @@ What is captured: the layer solves, the S-matrix chain and the R/T reduction
 (and, for GradientGraph, the adjoint sweep down to the pixel gradients),
 reading the sources from device buffers owned by the graph.  What stays
 outside: uploads of new sources (update_sources copies them into those
-buffers before a replay) and the status words of the eigensolver and the LU
-factorizations, which the captured sequence records instead of reading;
+buffers before a replay; a SolveGraph whose layers then want other doubling
+counts is captured again) and the status words of the layer solves and the
+star products, which the captured sequence records instead of reading;
 replay() checks them after the graph has run and raises numpy's LinAlgError
 as the eager call does.  Workspaces come from the graph's private memory pool
 and stay allocated while the graph object lives.  A replay overwrites the

@@ -118,7 +118,7 @@ class Layer:
 
     @property
     def patterned(self):
-        """True when the layer's modes come from the eigen-solver."""
+        """True for layers without closed-form modes (pixmaps, islands)."""
         return self.formulation in (Formulation.FFT, Formulation.ANALYTICAL)
 
     # ------------------------------------------------------------- solve
@@ -169,11 +169,11 @@ class Layer:
     @staticmethod
     def solve_batch_many(layers, kp, wl, rt_only=False, plan=None):
         """solve_batch for several layers of one expansion.  When all their
-        eigenproblems fit one round of the eigen-solver (khx_eig_slots), the
-        patterned layers are solved together in one fused call so that they
-        share the GPU (a single layer's small batch leaves most CUs idle); the
-        bound also keeps the fused workspace within one round's worth of
-        items.  plan: {id(layer): Doublings of its sources}, from plan_layers.
+        items fit one round of the eigen-solver (khx_eig_slots), the patterned
+        layers are solved together in one fused call so that they share the GPU
+        (a single layer's small batch leaves most CUs idle); the bound also
+        keeps the fused workspace within one round's worth of items, with modes
+        or without.  plan: {id(layer): Doublings of its sources}, from plan_layers.
         Everything else as solve_batch."""
         plan = plan or {}
         pat = [ly for ly in layers if getattr(ly, "patterned", False)]
