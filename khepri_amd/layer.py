@@ -333,11 +333,11 @@ def stack_layers(pw, layers, mask, reverse=True, ws=None, infos=None, solved=Fal
     spaces are the identity, its uniform layers diagonal scalings of a
     neighbour (a third of the star products of a typical stack are left).
     """
-    if solved and not reverse and not any(mask[1:-1]):
+    last = len(layers) - 1
+    if solved and not reverse and not any(mask[1:last]):
         Stot = _stack_forward(layers, ws, infos)
         if Stot is not None:
-            return [layers[0].S if mask[0] else None, *[None] * (len(layers) - 2), Stot if mask[-1] else None], \
-                None, Stot
+            return [layers[0].S if mask[0] else None, *[None] * (last - 1), Stot if mask[last] else None], None, Stot
     Stot = layers[0].S
     Sls = [Stot if mask[0] else None]
     for keep, layer in zip(mask[1:], layers[1:]):

@@ -101,6 +101,22 @@ def test_fold_is_for_layers_as_solved_by_the_library(monkeypatch):
         assert Stot is (layers[1].S if products == 0 else layers[0].S)
 
 
+def test_folded_stack_keeps_the_copies_the_mask_names(monkeypatch):
+    """The mask of a stack without half spaces (void crystal) is two longer than the
+    stack: its entry for the last layer decides, as it does without folding."""
+    from khepri_amd import Crystal
+    from khepri_amd.layer import Layer, stack_layers
+    e = Crystal((1, 1)).expansion
+    _recorded(monkeypatch)
+    layers = [Layer.uniform(e, 2.0, 0.3), Layer.uniform(e, 3.0, 0.3)]
+    for ly in layers:
+        ly.S = torch.zeros((1, 2, 2, 2, 2), dtype=torch.complex128)
+    for mask in ([True, False, False, True], [False, True], [True, True]):
+        copies = [[S is not None for S in stack_layers(None, layers, mask, reverse=False, solved=solved)[0]]
+                  for solved in (False, True)]
+        assert copies[0] == copies[1] == mask[:2]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["pixmap", "uniform"])
 def test_empty_batch(gpu, kind):
